@@ -129,39 +129,189 @@ __global__ void __launch_bounds__(256) local_cluster_kernel(LcArgs a)
                  [&](int dx, int dy) { return lc_read(a, y + dy, x + dx); });
 }
 
-// A 64 x 16 tile with a halo of `halo` = 2 (pntRange - 1) pixels (the walks'
-// reach) staged in LDS through lc_read, so every read the walks make sees
-// the byte the global-read kernel would.  Each thread filters 4 pixels of a
-// column (rows ty, ty + 4, ty + 8, ty + 12).
-constexpr int kLcTw = 64, kLcTh = 16;
+// A 64 x th tile with a halo of `halo` = 2 (pntRange - 1) pixels (the walks'
+// reach) staged in LDS by lc_read's address rule, so every read sees the
+// byte the global-read kernel would.
+//
+// The eight walks of a pixel end on their first step far more often than
+// not (noise sigma 10 against gap and diffe 10: four of five), and a walk
+// that ends there leaves the average at the centre's value.  With 1 <=
+// pntCount <= 8 the 8 - pntCount averages furthest from the centre are
+// replaced by it, so a pixel with no more surviving walks than that is
+// (8 cv - (8 - n) cv) / n = cv, exactly.  Phase 1 therefore only makes the
+// first step's two tests (integers: every operand is a sum of bytes, so the
+// comparisons are the floating ones), one pixel per lane, writes those
+// pixels and queues the others in LDS.  Phase 2 runs the queued pixels with
+// eight lanes each, one per direction, so that the walks of a pixel and of
+// its neighbours in the queue proceed together; the lanes' averages are
+// ranked and summed across the eight lanes with DPP moves.
+// Bound by VALU issue: one lane walking the eight directions of a pixel in
+// turn paid every direction's longest walk among 64 pixels and nine
+// divisions (about 1,290 issue slots per 64 pixels; 198 here, VALU 72% busy).
+// 2048 x 1536, pntRange 8, noise 10: 114 -> 26 us a call.  Eight waves per
+// workgroup measured 26.4 us, four 27.2, sixteen 35.3.
+constexpr int kLcTw = 64, kLcThMax = 64, kLcWaves = 8;
 constexpr int64_t kLcMaxLds = 48 * 1024;   // larger halos read global memory
 
-__global__ void __launch_bounds__(256) local_cluster_lds_kernel(LcArgs a, int halo)
+// value of lane (lane ^ X) within each group of eight lanes, X = 1..7
+template <int X>
+__device__ __forceinline__ int lc_xor8(int v)
 {
-    extern __shared__ uint8_t s_img[];
-    const int sw = kLcTw + 2 * halo, sh = kLcTh + 2 * halo;
-    const int x0 = blockIdx.x * kLcTw, y0 = blockIdx.y * kLcTh;
-    // row r of the tile is the linear range from (y0 - halo + r, x0 - halo),
-    // clamped byte by byte into the allocation as in lc_read
-    for (int r = threadIdx.x >> 6; r < sh; r += 4) {
+    if constexpr (X >= 4) v = __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true);   // lane ^ 7
+    constexpr int Q = X >= 4 ? (X ^ 7) : X;                                           // quad part
+    if constexpr (Q == 1) v = __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);
+    if constexpr (Q == 2) v = __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);
+    if constexpr (Q == 3) v = __builtin_amdgcn_mov_dpp(v, 0x1B, 0xF, 0xF, true);
+    return v;
+}
+
+// value of lane K of each quad
+template <int K>
+__device__ __forceinline__ float lc_quad_bcast(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xF, 0xF, true));
+}
+
+// 1 when lane ^ X is replaced before this lane: further from the centre
+// (distances as the bits of non-negative floats), or as far and later in
+// direction order (later = 1 when direction z ^ X comes after z).
+template <int X>
+__device__ __forceinline__ int lc_before(int dev, int later)
+{
+    return lc_xor8<X>(dev) + later > dev ? 1 : 0;
+}
+
+// SP: staged bytes per row (64 columns and both halos).
+template <int SP>
+__global__ void __launch_bounds__(64 * kLcWaves) local_cluster_lds_kernel(LcArgs a, int halo, int th)
+{
+    extern __shared__ __align__(16) uint8_t s_img[];
+    const int sh = th + 2 * halo;
+    uint16_t *queue = reinterpret_cast<uint16_t *>(s_img + SP * sh);
+    int *qcount = reinterpret_cast<int *>(queue + kLcTw * th);
+    const int x0 = blockIdx.x * kLcTw, y0 = blockIdx.y * th;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (threadIdx.x == 0) *qcount = 0;
+    // Row r of the tile is the linear range from (y0 - halo + r, x0 - halo).
+    // A row inside the allocation is read as aligned dwords (the second of a
+    // pair only where the row is misaligned: it then holds a wanted byte);
+    // any other is clamped byte by byte as in lc_read.
+    const int need = kLcTw + 2 * halo;                // bytes of a row that can be read
+    for (int r = wave; r < sh; r += kLcWaves) {
         const int64_t row = (int64_t)(y0 - halo + r) * a.pitch + (x0 - halo);
-        for (int c = threadIdx.x & 63; c < sw; c += 64) {
-            int64_t off = row + c;
-            off = off < a.lo ? a.lo : (off >= a.hi ? a.hi - 1 : off);
-            s_img[r * sw + c] = a.in[off];
+        if (row >= a.lo && row + SP <= a.hi) {
+            const uintptr_t p = reinterpret_cast<uintptr_t>(a.in + row);
+            const uint32_t mis = (uint32_t)(p & 3);
+            const uint32_t *src = reinterpret_cast<const uint32_t *>(p - mis);
+#pragma unroll
+            for (int c = lane; c < SP / 4; c += 64) {
+                const uint32_t lo = src[c], hi = src[c + (mis ? 1 : 0)];
+                *reinterpret_cast<uint32_t *>(s_img + r * SP + 4 * c) =
+                    __builtin_amdgcn_alignbyte(hi, lo, mis);
+            }
+        } else {
+            for (int c = lane; c < need; c += 64) {
+                int64_t off = row + c;
+                off = off < a.lo ? a.lo : (off >= a.hi ? a.hi - 1 : off);
+                s_img[r * SP + c] = a.in[off];
+            }
         }
     }
     __syncthreads();
-    const int x = x0 + (threadIdx.x & 63);
-    if (x >= a.W) return;
-#pragma unroll 1
-    for (int k = 0; k < kLcTh / 4; k++) {
-        const int y = y0 + (threadIdx.x >> 6) + 4 * k;
-        if (y >= a.H) break;
-        const int base = (y - y0 + halo) * sw + (x - x0 + halo);
-        a.out[(int64_t)y * a.out_pitch + x] =
-            lc_pixel(a, x, y, s_img[base],
-                     [&](int dx, int dy) { return (uint32_t)s_img[base + dy * sw + dx]; });
+    const uint32_t gap = (uint32_t)a.gap, diffe = (uint32_t)a.diffe;
+    // surviving walks a pixel may have and still be its own value
+    const int spare = a.pnt_count >= 1 && a.pnt_count <= 8 ? 8 - a.pnt_count : -1;
+    const int x = x0 + lane;
+    const bool xin = x >= a.pnt_range + 2 && x <= a.W - a.pnt_range - 2 && x < a.W;
+    const uint32_t gap_bias = 0x7FFFFFFFu - gap, diffe_bias = 0x7FFFFFFFu - diffe;
+    uint8_t *orow = a.out + (int64_t)(y0 + wave) * a.out_pitch + x;
+    for (int ly = wave; ly < th; ly += kLcWaves, orow += kLcWaves * a.out_pitch) {
+        const int y = y0 + ly;
+        if (y >= a.H) break;                          // whole waves
+        // the 5 x 5 window from its top-left corner
+        const uint8_t *w = s_img + (ly + halo - 2) * SP + lane + halo - 2;
+        const uint32_t cv = w[2 * SP + 2];
+        constexpr int dxs[8] = { 1, 1, 0, -1, -1, -1, 0, 1 }, dys[8] = { 0, -1, -1, -1, 0, 1, 1, 1 };
+        uint32_t n1[8], n2[8], ended = 0;
+#pragma unroll
+        for (int z = 0; z < 8; z++) {
+            n1[z] = w[(2 + dys[z]) * SP + 2 + dxs[z]];
+            n2[z] = w[(2 + 2 * dys[z]) * SP + 2 + 2 * dxs[z]];
+        }
+        // a test that fails carries its sum past 2^31: the larger sum's top
+        // bit says whether the walk ended
+#pragma unroll
+        for (int z = 0; z < 8; z++) {
+            const uint32_t g = __builtin_amdgcn_sad_u16(cv, n1[z], gap_bias);
+            const uint32_t d = __builtin_amdgcn_sad_u16(cv + n1[(z + 4) & 7], 2 * n2[z], diffe_bias);
+            ended = __builtin_amdgcn_alignbit(ended, g > d ? g : d, 31);
+        }
+        const int alive = a.pnt_range <= 1 ? 0 : 8 - __popc(ended);   // no steps: every average is cv
+        const bool more = xin && y >= a.pnt_range + 2 && y <= a.H - a.pnt_range - 2 &&
+                          (int)cv > a.pro_black && (int)cv < a.pro_white && alive > spare;
+        const uint64_t m = __ballot(more);
+        if (m) {
+            int at = 0;
+            if (lane == 0) at = atomicAdd(qcount, __popcll(m));
+            at = __builtin_amdgcn_readfirstlane(at);
+            const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+            if (more) queue[at + before] = (uint16_t)(ly * kLcTw + lane);
+        }
+        if (!more && x < a.W) *orow = (uint8_t)cv;
+    }
+    __syncthreads();
+    const int nq = __builtin_amdgcn_readfirstlane(*qcount);
+    const int z = lane & 7;                           // this lane's direction
+    const int zy = z == 0 || z == 4 ? 0 : (z < 4 ? -1 : 1);
+    const int zx = z == 2 || z == 6 ? 0 : (z < 2 || z == 7 ? 1 : -1);
+    const int dir = zy * SP + zx;
+    const int l1 = z & 1 ? 0 : 1, l2 = z & 2 ? 0 : 1, l4 = z & 4 ? 0 : 1;
+    for (int q0 = wave * 8; q0 < nq; q0 += 8 * kLcWaves) {      // whole waves
+        const int q = q0 + (lane >> 3);
+        const int e = queue[q < nq ? q : nq - 1];
+        int pos = (e / kLcTw + halo) * SP + (e & (kLcTw - 1)) + halo;
+        const uint32_t cv = s_img[pos];
+        const float fcv = (float)cv;
+        uint32_t cuv = s_img[pos + dir], pre1 = s_img[pos - dir], pre2 = cv;
+        uint32_t latt1 = s_img[pos + 2 * dir], sum = cv;
+        int i;
+        for (i = 1; i < a.pnt_range; i++) {
+            if (__builtin_amdgcn_sad_u16(cv, cuv, 0) > gap) break;
+            pos += 2 * dir;
+            const uint32_t latt2 = s_img[pos];
+            if (__builtin_amdgcn_sad_u16(pre1 + pre2, latt1 + latt2, 0) > diffe) break;
+            pre1 = pre2;
+            pre2 = cuv;
+            cuv = latt1;
+            latt1 = latt2;
+            sum += cuv;
+        }
+        float temp = (float)sum / (float)i;
+        const int dev = __float_as_int(fabsf(temp - fcv));
+        // Rounds that each replace the last of the furthest averages take
+        // them in (distance, direction) order: this lane's place in it.
+        const int rank = lc_before<1>(dev, l1) + lc_before<2>(dev, l2) + lc_before<3>(dev, l2) +
+                         lc_before<4>(dev, l4) + lc_before<5>(dev, l4) + lc_before<6>(dev, l4) +
+                         lc_before<7>(dev, l4);
+        if (rank < 8 - a.pnt_count) temp = fcv;
+        // the eight averages in direction order, from 0 (valid in lanes 0..3
+        // of each group)
+        const float rev = __int_as_float(lc_xor8<7>(__float_as_int(temp)));
+        float sumag = 0.0f;
+        sumag += lc_quad_bcast<0>(temp);
+        sumag += lc_quad_bcast<1>(temp);
+        sumag += lc_quad_bcast<2>(temp);
+        sumag += lc_quad_bcast<3>(temp);
+        sumag += lc_quad_bcast<3>(rev);
+        sumag += lc_quad_bcast<2>(rev);
+        sumag += lc_quad_bcast<1>(rev);
+        sumag += lc_quad_bcast<0>(rev);
+        sumag -= (float)((8 - a.pnt_count) * (int)cv);
+        const float v = sumag / (float)a.pnt_count;
+        if (z == 0 && q < nq)
+            a.out[(int64_t)(y0 + e / kLcTw) * a.out_pitch + x0 + (e & (kLcTw - 1))] =
+                v > 255.0f ? 255 : lc_sat_u8(v);
     }
 }
 
@@ -583,15 +733,31 @@ int bf_local_cluster(const bf_image_view *in, int64_t alloc_lo, int64_t alloc_hi
     a.diffe = (float)p->diffe_thred;
     a.pro_black = p->pro_black;
     a.pro_white = p->pro_white;
-    // the walks reach 2 (pntRange - 1) pixels from the centre, and 2 at least
+    // The walks reach 2 (pntRange - 1) pixels from the centre, and 2 at least.
+    // A halo whose 16-row tile exceeds the LDS bound reads global memory;
+    // the others take the tallest tile (fewer halo rows per pixel) that
+    // still gives every CU several workgroups.
     const int64_t halo = std::max<int64_t>(2, 2 * ((int64_t)a.pnt_range - 1));
-    const int64_t lds = (kLcTw + 2 * halo) * (kLcTh + 2 * halo);
-    if (lds <= kLcMaxLds)
-        hipLaunchKernelGGL(local_cluster_lds_kernel, dim3((a.W + kLcTw - 1) / kLcTw, (a.H + kLcTh - 1) / kLcTh),
-                           dim3(256), (size_t)lds, (hipStream_t)stream, a, (int)halo);
-    else
+    if ((kLcTw + 2 * halo) * (16 + 2 * halo) > kLcMaxLds) {
         hipLaunchKernelGGL(local_cluster_kernel, dim3((a.W + 63) / 64, (a.H + 3) / 4), dim3(256), 0,
                            (hipStream_t)stream, a);
+    } else {
+        // staged row: 64 columns and two halos, as one of three compiled
+        // pitches (halo <= 16, 32 and 96 pixels)
+        const int sp = halo <= 16 ? 96 : (halo <= 32 ? 128 : 256);
+        int cus = 0;
+        BF_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, current_device()));
+        const int64_t tx = (a.W + kLcTw - 1) / kLcTw;
+        auto lds_of = [&](int rows) {
+            return (size_t)sp * (rows + 2 * halo) + sizeof(uint16_t) * kLcTw * rows + sizeof(int);
+        };
+        int th = kLcThMax;
+        while (th > 16 && (tx * ((a.H + th - 1) / th) < 4 * (int64_t)cus || lds_of(th) > 64 * 1024)) th /= 2;
+        const dim3 grid((unsigned)tx, (a.H + th - 1) / th);
+        const auto kern = sp == 96 ? local_cluster_lds_kernel<96>
+                                   : (sp == 128 ? local_cluster_lds_kernel<128> : local_cluster_lds_kernel<256>);
+        hipLaunchKernelGGL(kern, grid, dim3(64 * kLcWaves), lds_of(th), (hipStream_t)stream, a, (int)halo, th);
+    }
     BF_HIP(hipGetLastError());
     return kOk;
 }
