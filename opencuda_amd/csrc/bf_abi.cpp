@@ -221,26 +221,24 @@ static int tiles_of(const DevJob &j, int config)
 }
 
 // Switch a job to the canonical per-q table of the unrolled kernels when
-// the template is the canonical ring, it holds the radius's taps and the
-// table fits next to a `config` tile with `halo`.
+// the template is the canonical ring and holds the radius's taps.  Rows that
+// do not fit in LDS beside a `config` tile with `halo` stay with job.rowg.
 bool ring_job(const Lut *L, int radius, int mode, int config, int halo, DevJob *job)
 {
     const int rr = ring_rows(radius, mode);
-    if (!L->canonical || rr <= 0 || ntaps_for(radius, mode) > L->count || job->sep ||
-        halo < halo_class(radius) || lds_bytes(config, halo, rr + 1) > max_lds_bytes())
+    if (!L->canonical || rr <= 0 || ntaps_for(radius, mode) > L->count || halo < halo_class(radius))
         return false;
+    const int fused = std::min(rr, ring_fused(config, halo));
     job->rowg = L->d_rowq;
-    job->nrows = rr;
-    job->lut_rows = rr + 1;
+    job->sep = 0;
+    job->nrows = fused;
+    job->erow = fused < rr ? 1 : 0;
+    job->xrow = ring_extra_row(radius);
+    job->lut_rows = fused + 1;
     // LDS key as make_job forms it: with one weight per q the per-q table
     // equals the per-weight one whenever their row counts agree
     job->lut_key = (L->id << 12) | (rr << 1);
     return true;
-}
-
-bool ring64_job(const Lut *L, int radius, int mode, DevJob *job)
-{
-    return ring64_available(radius) && ring_job(L, radius, mode, 0, halo_class(radius), job);
 }
 
 bool views_overlap(const bf_image_view *a, const bf_image_view *b)
@@ -477,9 +475,7 @@ int bf_exact(const bf_image_view *in, const bf_image_view *out, bf_lut lut, int3
         return kNullPointer;
     }
     Lut *L = lut_from_handle(lut);
-    int rcfg = -1;
-    if (L->canonical && ring_available(radius, mode, &rcfg) && ring_rows(radius, mode) > 0 &&
-        ntaps_for(radius, mode) <= L->count) {
+    if (L->canonical && ring_rows(radius, mode) > 0 && ntaps_for(radius, mode) <= L->count) {
         if (!in || !out) {
             set_error("null argument");
             return kNullPointer;
@@ -489,15 +485,17 @@ int bf_exact(const bf_image_view *in, const bf_image_view *out, bf_lut lut, int3
             set_error("input and output views overlap");
             return kInvalidData;
         }
+        const int rcfg = ring_config(radius, mode, std::min(in->width, out->width),
+                                     std::min(in->height, out->height));
         DevJob job;
-        int rc = make_job(in, out, L, radius, mode, rcfg, halo_class(radius), 0, &job, nullptr);
+        int rc = make_job(in, out, L, radius, mode, std::max(rcfg, 0), halo_class(radius), 0, &job, nullptr);
         if (rc) return rc;
-        if (ring_job(L, radius, mode, rcfg, halo_class(radius), &job))
-            return launch_ring(job, radius, mode, tiles_of(job, rcfg), (hipStream_t)stream);
+        if (rcfg >= 0 && ring_job(L, radius, mode, rcfg, halo_class(radius), &job))
+            return launch_ring(job, rcfg, tiles_of(job, rcfg), nullptr, nullptr, (hipStream_t)stream);
     }
     const int rows = fused_rows(lut_from_handle(lut), radius, mode);
     const int tuned = tuned_config(radius, mode);
-    const int want = tuned >= 0 ? tuned : default_config(radius, mode);
+    const int want = tuned >= 0 ? tuned : (radius >= 17 ? 3 : default_config(radius, mode));
     const int config = rows < 0 ? default_config(1, mode) : fit_config(want, radius, rows);
     return bf_exact_config(in, out, lut, radius, mode, config, stream);
 }
@@ -533,7 +531,7 @@ int bf_tune_radius(int32_t radius, int32_t mode, int32_t width, int32_t height, 
     bf_image_view vin{ din, width, height, width }, vout{ dout, width, height, width };
     // Each configuration is timed as a one-job batch: the launch a batch
     // with that configuration makes (the unrolled kernels where they apply,
-    // configurations 0 and 1 at r = 3, 5, 7, 9, 15; the tap-list kernel
+    // configurations 0 and 1 to r = 16; the tap-list kernel
     // otherwise), which is what the table's costs steer.
     const bf_job job{ vin, vout, lut, radius, mode };
     for (int c = 0; c < nc && rc == kOk; c++) {

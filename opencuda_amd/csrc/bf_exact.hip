@@ -38,9 +38,18 @@
 #include <utility>
 
 #include "bf_internal.h"
+#include "bf_ring.h"
 #include "bf_tile.h"
 
 namespace bfimpl {
+
+BF_RING_SMALL(extern, 0)
+BF_RING_MID(extern, 0)
+BF_RING_LARGE(extern, 0)
+BF_RING_SMALL(extern, 1)
+BF_RING_MID(extern, 1)
+BF_RING_LARGE(extern, 1)
+BF_RING_STD_LARGE(extern)
 
 namespace {
 
@@ -96,7 +105,7 @@ __device__ __forceinline__ void tile_ref(const DevJob &job, int X0, int Y0, int 
     for (int j = 0; j < CPL; j++) {
         const int x = X0 + CPL * lx + j;
         if (x < job.W) {
-            uint8_t *o = job.out + (int64_t)y0 * job.out_pitch + x;
+            BF_GLOBAL uint8_t *o = as_global(job.out) + (int64_t)y0 * job.out_pitch + x;
 #pragma unroll
             for (int k = 0; k < 4; k++)
                 if (y0 + k < job.H) o[k * job.out_pitch] = to_u8(t[k][j] / sum[k][j]);
@@ -150,7 +159,7 @@ __device__ __forceinline__ void tile_std(const DevJob &job, int X0, int Y0, int 
     for (int j = 0; j < CPL; j++) {
         const int x = X0 + CPL * lx + j;
         if (x < job.W) {
-            uint8_t *o = job.out + (int64_t)y0 * job.out_pitch + x;
+            BF_GLOBAL uint8_t *o = as_global(job.out) + (int64_t)y0 * job.out_pitch + x;
 #pragma unroll
             for (int k = 0; k < 4; k++)
                 if (y0 + k < job.H) o[k * job.out_pitch] = to_u8(t[k][j] / sum[k][j]);
@@ -216,30 +225,6 @@ bf_exact_kernel(KArgs args)
             else
                 tile_std<TW, TGY, HALO, CPL, false>(job, X0, Y0, lx, gy);
         }
-    }
-}
-
-// One image, static grid-stride over its tiles (or over the tiles of a
-// device list, whose length is read on the device); job.rowg holds the
-// per-q weights of the canonical template and job.nrows their count.
-template <int R, int MODE, int TW, int TGY, int HALO>
-__global__ void __launch_bounds__(TW * TGY)
-bf_ring_kernel(DevJob job, int ntiles, const int32_t *list, const int32_t *list_count)
-{
-    using G = Geo<TW, TGY, HALO>;
-    const int tid = threadIdx.x;
-    const int lx = tid % TW, gy = tid / TW;
-    build_lut<G::NT>(job, kTileOff + (uint32_t)G::TILE_BYTES, tid);
-    const int n = list ? *as_const(list_count) : ntiles;
-    for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        const int tile = list ? as_const(list)[i] : i;
-        const int ty = tile / job.tiles_x;
-        const int X0 = (tile - ty * job.tiles_x) * TW;
-        const int Y0 = ty * G::TH;
-        __syncthreads();                      // table built / previous tile consumed
-        load_tile<TW, TGY, HALO>(job, X0, Y0, tid);
-        __syncthreads();
-        tile_ring<R, MODE, TW, TGY, HALO>(job, X0, Y0, lx, gy);
     }
 }
 
@@ -338,15 +323,15 @@ __global__ void __launch_bounds__(64) check_kernel(CheckArgs a)
 // share a CU (the taps' LDS latency needs the waves).
 constexpr int kCheckGroup = 8;            // taps per scheduling window (4 to 32 measured alike)
 
-template <int R, int MODE, int HALO>
+template <int MODE, int HALO>
 __global__ void __launch_bounds__(256) ring_check_kernel(CheckArgs a, int ntiles)
 {
     constexpr int SPAN = 64 + 2 * HALO;
     constexpr uint32_t WIN = SPAN * SPAN;
     constexpr uint32_t E_BASE = kTileOff + 4 * WIN;
-    constexpr int T = RingTaps<R, MODE>::T;
-    constexpr int MINB = ring_min_offset<R, MODE, SPAN>();
+    constexpr int MINB = ring_min_offset<HALO, SPAN>();
     const DevJob &j = a.job;
+    const int radius = __builtin_amdgcn_readfirstlane(j.radius);
     const int tid = threadIdx.x, wave = tid >> 6, cell = tid & 63;
     const uint32_t win = kTileOff + (uint32_t)wave * WIN;
     for (int d = tid; d < 256; d += 256) lds_store_u32(E_BASE + 4 * d, __float_as_uint(j.range[d]));
@@ -370,8 +355,8 @@ __global__ void __launch_bounds__(256) ring_check_kernel(CheckArgs a, int ntiles
             const uint32_t c4 = lds_u8(win + (uint32_t)((sy + HALO) * SPAN + sx + HALO)) * 0x01010101u;
             const uint32_t tbase = win + (uint32_t)((wy + HALO) * SPAN + sx + HALO + MINB);
             float t = 0.0f, s = 0.0f;
-            static_for<T>([&](auto ci) {
-                constexpr RingTap tp = kRing<R, MODE>.t[decltype(ci)::value];
+            auto tap = [&](auto ci) __attribute__((always_inline)) {
+                constexpr RingTap tp = kRing<HALO>.t[decltype(ci)::value];
                 constexpr int TAPB = tp.dy * SPAN + tp.dx - MINB;   // >= 0
                 const uint32_t p = lds_u8(tbase + TAPB);
                 // v_perm_b32 with selector 0 replicates byte 0 (one full-rate op)
@@ -380,9 +365,28 @@ __global__ void __launch_bounds__(256) ring_check_kernel(CheckArgs a, int ntiles
                 const float f = j.rowg[tp.row] * e;
                 t = t + f * (float)(p4 & 0xFFu);
                 s = s + f;
-                if constexpr (decltype(ci)::value % kCheckGroup == kCheckGroup - 1)
-                    asm volatile("" : "+v"(t), "+v"(s)::"memory");
+            };
+            auto fence = [&]() __attribute__((always_inline)) {
+                asm volatile("" : "+v"(t), "+v"(s)::"memory");
+            };
+            // ring by ring, as tile_ring
+            tap(std::integral_constant<int, 0>{});
+            static_for<HALO>([&](auto ri) {
+                constexpr int I = decltype(ri)::value + 1, C0 = ring_first(I), N = 8 * I;
+                if constexpr (I > halo_min_radius(HALO))
+                    if (radius < I) return;
+                static_for<N>([&](auto ci) {
+                    constexpr int C = C0 + decltype(ci)::value;
+                    tap(std::integral_constant<int, C>{});
+                    if constexpr (C % kCheckGroup == kCheckGroup - 1) fence();
+                });
             });
+            if constexpr (MODE == kModeRef) {
+                const uint32_t p4 = lds_u8(win + (uint32_t)((wy + HALO + radius + 1) * SPAN + sx + HALO - radius)) * 0x01010101u;
+                const float f = j.rowg[j.xrow] * lds_f32(__builtin_amdgcn_sad_u8(p4, c4, E_BASE));
+                t = t + f * (float)(p4 & 0xFFu);
+                s = s + f;
+            }
             const int ex = to_u8(t / s);
             const int su = j.out[(int64_t)y * j.out_pitch + x];
             bad = (ex - su > a.tol) || (su - ex > a.tol);
@@ -521,31 +525,10 @@ int exact_tiles(const DevJob &job, const int32_t *tile_list_dev, int ntiles_max,
 
 namespace {
 
-template <int R, int MODE, int TW, int TGY, int HALO>
-int launch_ring_one(const DevJob &job, int ntiles, const int32_t *list, const int32_t *count,
-                    hipStream_t s)
-{
-    using G = Geo<TW, TGY, HALO>;
-    constexpr auto kern = bf_ring_kernel<R, MODE, TW, TGY, HALO>;
-    const size_t lds = kTileOff + (size_t)G::TILE_BYTES + (size_t)(job.nrows + 1) * 1024;
-    BF_HIP(allow_full_lds<kern>());
-    const int res = resident_groups(reinterpret_cast<const void *>(kern), G::NT, lds);
-    if (res < 0) return hip_fail(hipGetLastError(), "occupancy query");
-    if (res < 1) {
-        set_error("ring kernel does not fit on a CU");
-        return kInvalidData;
-    }
-    const int grid = std::min(ntiles, res);   // with a list, ntiles = its maximum length
-    if (grid < 1) return kOk;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(G::NT), lds, s, job, ntiles, list, count);
-    BF_HIP(hipGetLastError());
-    return kOk;
-}
-
-template <int R, int MODE, int HALO>
+template <int MODE, int HALO>
 int launch_ring_check_one(const CheckArgs &a, int ntiles, hipStream_t s)
 {
-    constexpr auto kern = ring_check_kernel<R, MODE, HALO>;
+    constexpr auto kern = ring_check_kernel<MODE, HALO>;
     const size_t lds = kTileOff + 4 * (size_t)(64 + 2 * HALO) * (64 + 2 * HALO) + 1024;
     BF_HIP(allow_full_lds<kern>());
     const int res = resident_groups(reinterpret_cast<const void *>(kern), 256, lds);
@@ -563,84 +546,102 @@ int launch_ring_check_one(const CheckArgs &a, int ntiles, hipStream_t s)
 
 }  // namespace
 
-bool ring_available(int radius, int mode, int *config)
+// Tile config of a single image.  Both shapes hold the same lanes per SIMD
+// while two 64 x 32 workgroups fit a CU beside their tables (r <= 9).  Above,
+// a CU runs one workgroup, and a 64 x 32 tile takes about 0.6 of a 64 x 64
+// one's time (its two waves a SIMD cover less latency): it wins where halving
+// the tiles does not add rounds, on images of up to about 700^2 (640 x 480,
+// r = 14 REF: 75 against 125 us).
+// REF from r = 17 forms many factors per tap here too, and below 12 Mpix the
+// tap list on 64 x 16 tiles, whose small table leaves room for several
+// workgroups a CU, fills the last round better (1500 x 1100, r = 18: 318
+// against 379 us; 3000^2, r = 17: 1.31 against 1.35 ms; 4096^2: 2.45 against
+// 2.32): -1.
+int ring_config(int radius, int mode, int W, int H)
 {
-    switch (radius) {
-    case 15: *config = 0; return true;
-    case 3: case 5: case 7: case 9: *config = 1; return true;
-    default: (void)mode; return false;
-    }
+    if (radius <= 9) return 1;
+    if (mode == kModeRef && radius >= 17) return (int64_t)W * H < 12000000 ? -1 : 0;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        return 0;
+    const int64_t tx = (W + 63) / 64, t64 = tx * ((H + 63) / 64), t32 = tx * ((H + 31) / 32);
+    return 6 * ((t32 + cus - 1) / cus) < 10 * ((t64 + cus - 1) / cus) ? 1 : 0;
 }
+
+// 64 x 64 tiles also serve tile lists (the surrogate's fallback) from r = 9.
+bool ring_kernel_available(int radius, int mode, int config)
+{
+    if (radius < 1 || radius > BF_MAX_RADIUS) return false;
+    return config == 0 ? radius >= 9 : (config == 1 && (mode != kModeRef || radius <= 16));
+}
+
+static constexpr RingTaps<BF_MAX_RADIUS> kAllRings;
 
 int ring_rows(int radius, int mode)
 {
-    switch (radius * 2 + (mode == kModeRef ? 0 : 1)) {
-    case 30: return RingTaps<15, 0>().nrows;
-    case 31: return RingTaps<15, 1>().nrows;
-    case 6: return RingTaps<3, 0>().nrows;
-    case 7: return RingTaps<3, 1>().nrows;
-    case 10: return RingTaps<5, 0>().nrows;
-    case 11: return RingTaps<5, 1>().nrows;
-    case 14: return RingTaps<7, 0>().nrows;
-    case 15: return RingTaps<7, 1>().nrows;
-    case 18: return RingTaps<9, 0>().nrows;
-    case 19: return RingTaps<9, 1>().nrows;
-    default: return -1;
-    }
+    if (radius < 1 || radius > BF_MAX_RADIUS) return -1;
+    return mode == kModeRef ? std::max(kAllRings.rows[radius], kAllRings.xrow[radius] + 1)
+                            : kAllRings.rows[radius];
 }
 
-int launch_ring(const DevJob &job, int radius, int mode, int ntiles, hipStream_t s)
+int ring_extra_row(int radius) { return kAllRings.xrow[radius]; }
+
+int ring_fused(int config, int halo)
 {
-    const bool ref = mode == kModeRef;
-    switch (radius) {
-    case 15: return ref ? launch_ring_one<15, 0, 64, 16, 16>(job, ntiles, nullptr, nullptr, s)
-                        : launch_ring_one<15, 1, 64, 16, 16>(job, ntiles, nullptr, nullptr, s);
-    case 9: return ref ? launch_ring_one<9, 0, 64, 8, 12>(job, ntiles, nullptr, nullptr, s)
-                       : launch_ring_one<9, 1, 64, 8, 12>(job, ntiles, nullptr, nullptr, s);
-    case 7: return ref ? launch_ring_one<7, 0, 64, 8, 8>(job, ntiles, nullptr, nullptr, s)
-                       : launch_ring_one<7, 1, 64, 8, 8>(job, ntiles, nullptr, nullptr, s);
-    case 5: return ref ? launch_ring_one<5, 0, 64, 8, 8>(job, ntiles, nullptr, nullptr, s)
-                       : launch_ring_one<5, 1, 64, 8, 8>(job, ntiles, nullptr, nullptr, s);
-    case 3: return ref ? launch_ring_one<3, 0, 64, 8, 4>(job, ntiles, nullptr, nullptr, s)
-                       : launch_ring_one<3, 1, 64, 8, 4>(job, ntiles, nullptr, nullptr, s);
-    default: set_error("no unrolled kernel for this radius"); return kInvalidData;
-    }
+    const TileConfig &c = kConfigs[config];
+    return (int)((max_lds_bytes() - kTileOff - (size_t)(c.tw + 2 * halo) * (4 * c.tgy + 2 * halo) * 4) / 1024) - 1;
 }
 
-bool ring64_available(int radius) { return radius == 15 || radius == 9; }
-
-int ring64_tiles(const DevJob &job, int radius, int mode, const int32_t *list,
-                 const int32_t *count, int ntiles_max, hipStream_t s)
+int launch_ring(const DevJob &job, int config, int ntiles, const int32_t *list, const int32_t *count,
+                hipStream_t s)
 {
-    const bool ref = mode == kModeRef;
-    switch (radius) {
-    case 15: return ref ? launch_ring_one<15, 0, 64, 16, 16>(job, ntiles_max, list, count, s)
-                        : launch_ring_one<15, 1, 64, 16, 16>(job, ntiles_max, list, count, s);
-    case 9: return ref ? launch_ring_one<9, 0, 64, 16, 12>(job, ntiles_max, list, count, s)
-                       : launch_ring_one<9, 1, 64, 16, 12>(job, ntiles_max, list, count, s);
-    default: set_error("no unrolled 64x64 kernel for this radius"); return kInvalidData;
+    if (!ring_kernel_available(job.radius, job.mode, config)) {
+        set_error("no unrolled kernel for this radius and tile config");
+        return kInvalidData;
     }
-}
-
-int launch_check(const CheckArgs &a, int ring_radius, int ntiles, hipStream_t s)
-{
-    const bool ref = a.job.mode == kModeRef;
-    switch (ring_radius) {
-    case 15: return ref ? launch_ring_check_one<15, 0, 16>(a, ntiles, s)
-                        : launch_ring_check_one<15, 1, 16>(a, ntiles, s);
-    case 9: return ref ? launch_ring_check_one<9, 0, 12>(a, ntiles, s)
-                       : launch_ring_check_one<9, 1, 12>(a, ntiles, s);
-    case 0:
-        if (a.halo < 0 || a.halo > kCheckHaloMax) {
-            set_error("radius outside the check kernel's halo");
-            return kInvalidData;
+    const bool ref = job.mode == kModeRef;
+    if (config == 1) {
+        switch (halo_class(job.radius)) {
+        case 4: return ref ? launch_ring_one<0, 64, 8, 4>(job, ntiles, list, count, s)
+                           : launch_ring_one<1, 64, 8, 4>(job, ntiles, list, count, s);
+        case 8: return ref ? launch_ring_one<0, 64, 8, 8>(job, ntiles, list, count, s)
+                           : launch_ring_one<1, 64, 8, 8>(job, ntiles, list, count, s);
+        case 12: return ref ? launch_ring_one<0, 64, 8, 12>(job, ntiles, list, count, s)
+                            : launch_ring_one<1, 64, 8, 12>(job, ntiles, list, count, s);
+        case 16: return ref ? launch_ring_one<0, 64, 8, 16>(job, ntiles, list, count, s)
+                            : launch_ring_one<1, 64, 8, 16>(job, ntiles, list, count, s);
+        default: return launch_ring_one<1, 64, 8, 20>(job, ntiles, list, count, s);
         }
-        if (ntiles < 1) return kOk;
-        hipLaunchKernelGGL(check_kernel, dim3(ntiles), dim3(64), 0, s, a);
-        BF_HIP(hipGetLastError());
-        return kOk;
-    default: set_error("no unrolled check kernel for this radius"); return kInvalidData;
     }
+    switch (halo_class(job.radius)) {
+    case 12: return ref ? launch_ring_one<0, 64, 16, 12>(job, ntiles, list, count, s)
+                        : launch_ring_one<1, 64, 16, 12>(job, ntiles, list, count, s);
+    case 16: return ref ? launch_ring_one<0, 64, 16, 16>(job, ntiles, list, count, s)
+                        : launch_ring_one<1, 64, 16, 16>(job, ntiles, list, count, s);
+    default: return ref ? launch_ring_one<0, 64, 16, 20>(job, ntiles, list, count, s)
+                        : launch_ring_one<1, 64, 16, 20>(job, ntiles, list, count, s);
+    }
+}
+
+bool ring_check_available(int radius) { return radius >= 9 && radius <= 16; }
+
+int launch_check(const CheckArgs &a, bool ring, int ntiles, hipStream_t s)
+{
+    if (ring) {
+        const bool ref = a.job.mode == kModeRef;
+        if (a.job.radius > 12)
+            return ref ? launch_ring_check_one<0, 16>(a, ntiles, s) : launch_ring_check_one<1, 16>(a, ntiles, s);
+        return ref ? launch_ring_check_one<0, 12>(a, ntiles, s) : launch_ring_check_one<1, 12>(a, ntiles, s);
+    }
+    if (a.halo < 0 || a.halo > kCheckHaloMax) {
+        set_error("radius outside the check kernel's halo");
+        return kInvalidData;
+    }
+    if (ntiles < 1) return kOk;
+    hipLaunchKernelGGL(check_kernel, dim3(ntiles), dim3(64), 0, s, a);
+    BF_HIP(hipGetLastError());
+    return kOk;
 }
 
 int launch_reset_counter(int *counter, hipStream_t s)

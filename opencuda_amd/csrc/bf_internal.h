@@ -83,6 +83,8 @@ struct alignas(16) DevJob {
     int32_t sep;             // 1: LDS holds E only, g*E formed per tap (large radii)
     int32_t lut_rows;        // 1 KB rows of the LDS table: nrows + 1, or 1 when sep
     int32_t radius;
+    int32_t erow;            // 1: row nrows holds E (unrolled kernels, rows past LDS)
+    int32_t xrow;            // unrolled kernels: table row of REF's extra tap
 };
 
 struct TileConfig {
@@ -108,9 +110,8 @@ size_t max_lds_bytes();
 //             grid-stride schedule.
 int launch_exact(int config, int halo, const DevJob &job0, const DevJob *jobs_dev,
                  int njobs, int ntiles, int max_lut_rows, int *counter, hipStream_t s);
-// The same launch for jobs that all use the canonical template at radii
-// with unrolled kernels (3, 5, 7, 9, 15; tables from ring_job), tile
-// configs 0 and 1, halo <= 16.
+// The same launch for jobs that all use the canonical template (tables from
+// ring_job), tile configs 0 and 1, halo <= 16.
 bool ring_batch_supported(int config, int halo);
 int launch_ring_batch(int config, int halo, const DevJob *jobs_dev, int njobs, int ntiles,
                       int max_lut_rows, int *counter, hipStream_t s);
@@ -125,11 +126,17 @@ int make_job(const bf_image_view *in, const bf_image_view *out, const Lut *lut,
 // exceeds the template.
 int fused_rows(const Lut *lut, int radius, int mode);
 
-// Unrolled kernels for the canonical ring template: which radii have one
-// (and the tile config they use), their fused-table row count, the launch.
-bool ring_available(int radius, int mode, int *config);
+// Unrolled kernels for the canonical ring template: the tile config a radius
+// runs best with on a W x H image (-1: the tap-list kernel), the table rows of a radius, the row of REF's extra tap, the
+// configs with a kernel, how many rows LDS holds, the launch (over all tiles,
+// or over a device list of at most ntiles tiles).
+int ring_config(int radius, int mode, int W, int H);
 int ring_rows(int radius, int mode);
-int launch_ring(const DevJob &job, int radius, int mode, int ntiles, hipStream_t s);
+int ring_extra_row(int radius);
+bool ring_kernel_available(int radius, int mode, int config);
+int ring_fused(int config, int halo);
+int launch_ring(const DevJob &job, int config, int ntiles, const int32_t *list, const int32_t *count,
+                hipStream_t s);
 
 Lut *lut_from_handle(bf_lut h);
 int current_device();
@@ -140,16 +147,10 @@ bool views_overlap(const bf_image_view *a, const bf_image_view *b);
 int exact_tiles(const DevJob &job, const int32_t *tile_list_dev, int ntiles_dev_max,
                 const int32_t *count_dev, int config, int halo, hipStream_t s);
 
-// Unrolled kernels on 64x64 tiles (the surrogate's check and fallback
-// tiles) for the canonical template at these radii.  ring64_job switches a
-// job made for config 0 to the canonical per-q table when they apply.
-bool ring64_available(int radius);
-bool ring64_job(const Lut *lut, int radius, int mode, DevJob *job);
-// Switch a job (made for `config` with `halo`) to the canonical per-q
-// table of the unrolled kernels; false (job unchanged) when they do not apply.
+// Switch a job made for `config` with `halo` to the canonical per-q table of
+// the unrolled kernels; false (job unchanged) when the template is not the
+// canonical one or does not hold the radius.
 bool ring_job(const Lut *lut, int radius, int mode, int config, int halo, DevJob *job);
-int ring64_tiles(const DevJob &job, int radius, int mode, const int32_t *list,
-                 const int32_t *count, int ntiles_max, hipStream_t s);
 
 // Exact sample check of 64x64 tiles (one hashed sample per 8x8 cell).
 struct CheckArgs {
@@ -164,8 +165,9 @@ struct CheckArgs {
     uint32_t salt;
     int halo;                    // context rows/columns staged around a tile
 };
-// ring_radius 0: the run-time tap list; 9 or 15: the unrolled canonical
-// template (job from ring64_job).
-int launch_check(const CheckArgs &a, int ring_radius, int ntiles, hipStream_t s);
+// ring: the unrolled canonical template (job from ring_job) where the radius
+// has such a kernel, else the run-time tap list.
+bool ring_check_available(int radius);
+int launch_check(const CheckArgs &a, bool ring, int ntiles, hipStream_t s);
 
 }  // namespace bfimpl

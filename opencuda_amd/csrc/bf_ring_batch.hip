@@ -1,8 +1,8 @@
 // bf_ring_batch.hip -- batches of jobs on the canonical (GAUSS-factory)
 // template, TemplateFactory.cu:1092-1168: the persistent work-queue launch
-// of bf_exact_kernel, with each tile filtered by the unrolled kernel of its
-// job's radius and mode (tap offsets and table rows compiled in) instead of
-// the run-time tap list.  Results are the same bits; the batch only saves
+// of bf_exact_kernel, with each tile filtered by the unrolled tap list of its
+// job's mode up to the job's radius (tap offsets and table rows compiled in)
+// instead of the run-time tap list.  Results are the same bits; the batch only saves
 // the tap-list decoding.
 #include <hip/hip_runtime.h>
 
@@ -15,15 +15,10 @@ namespace bfimpl {
 
 namespace {
 
-// One unrolled radius: instantiated only where the staged halo covers it.
-template <int R, int MODE, int TW, int TGY, int HALO>
-__device__ __forceinline__ void ring_if_fits(const DevJob &job, int X0, int Y0, int lx, int gy)
-{
-    if constexpr (R <= HALO) tile_ring<R, MODE, TW, TGY, HALO>(job, X0, Y0, lx, gy);
-}
-
+// Registers for six waves a SIMD where the tables of the radii leave room for
+// three workgroups (r <= 8 on 64 x 32 tiles), for four elsewhere.
 template <int TW, int TGY, int HALO>
-__global__ void __launch_bounds__(TW * TGY) bf_ring_batch_kernel(KArgs args)
+__global__ void __launch_bounds__(TW * TGY, HALO <= 8 && TGY == 8 ? 6 : 4) bf_ring_batch_kernel(KArgs args)
 {
     using G = Geo<TW, TGY, HALO>;
     const int tid = threadIdx.x;
@@ -55,19 +50,10 @@ __global__ void __launch_bounds__(TW * TGY) bf_ring_batch_kernel(KArgs args)
         }
         load_tile<TW, TGY, HALO>(job, X0, Y0, tid);
         __syncthreads();
-        switch (job.radius * 2 + (job.mode == kModeRef ? 0 : 1)) {
-        case 6: ring_if_fits<3, 0, TW, TGY, HALO>(job, X0, Y0, lx, gy); break;
-        case 7: ring_if_fits<3, 1, TW, TGY, HALO>(job, X0, Y0, lx, gy); break;
-        case 10: ring_if_fits<5, 0, TW, TGY, HALO>(job, X0, Y0, lx, gy); break;
-        case 11: ring_if_fits<5, 1, TW, TGY, HALO>(job, X0, Y0, lx, gy); break;
-        case 14: ring_if_fits<7, 0, TW, TGY, HALO>(job, X0, Y0, lx, gy); break;
-        case 15: ring_if_fits<7, 1, TW, TGY, HALO>(job, X0, Y0, lx, gy); break;
-        case 18: ring_if_fits<9, 0, TW, TGY, HALO>(job, X0, Y0, lx, gy); break;
-        case 19: ring_if_fits<9, 1, TW, TGY, HALO>(job, X0, Y0, lx, gy); break;
-        case 30: ring_if_fits<15, 0, TW, TGY, HALO>(job, X0, Y0, lx, gy); break;
-        case 31: ring_if_fits<15, 1, TW, TGY, HALO>(job, X0, Y0, lx, gy); break;
-        default: break;                            // excluded by the host (ring_job)
-        }
+        if (job.mode == kModeRef)
+            tile_ring<0, TW, TGY, HALO, 1, ring_group<0, HALO, true>()>(job, X0, Y0, lx, gy);
+        else
+            tile_ring<1, TW, TGY, HALO, 1, ring_group<1, HALO, true>()>(job, X0, Y0, lx, gy);
     }
 }
 

@@ -1,0 +1,6 @@
+// bf_ring_ref_mid.hip -- instances of the unrolled REF kernels (bf_ring.h).
+#include "bf_ring.h"
+
+namespace bfimpl {
+BF_RING_MID(, 0)
+}  // namespace bfimpl

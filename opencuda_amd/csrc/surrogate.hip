@@ -1922,12 +1922,15 @@ static int sur_filter(Net *net, const bf_image_view *in, const bf_image_view *ou
     }
     hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, s, ws.count, 1);
     BF_HIP(hipGetLastError());
-    // The canonical template at r = 9 or 15 runs the unrolled 64x64-tile
-    // kernels for both the check and the fallback (same taps, order and
+    // The canonical template runs the unrolled 64x64-tile kernels from r = 9
+    // for the fallback, and to r = 16 for the check too (same taps, order and
     // rounding as the run-time tap list, so the same verdicts and pixels).
-    const bool ring = ring64_job(lut_from_handle(lut), radius, mode, &job);
+    DevJob rjob = job;
+    const bool ring = ring_kernel_available(radius, mode, 0) &&
+                      ring_job(lut_from_handle(lut), radius, mode, 0, halo_class(radius), &rjob);
+    const bool ring_check = ring && ring_check_available(radius);
     CheckArgs ca{};
-    ca.job = job;
+    ca.job = ring_check ? rjob : job;
     ca.rowg = lut_from_handle(lut)->d_rowg;
     ca.tiles_x = tx;
     ca.tiles_y = ty;
@@ -1940,9 +1943,9 @@ static int sur_filter(Net *net, const bf_image_view *in, const bf_image_view *ou
     // make_job has checked every tap against this halo (REF rows may reach
     // two further down, which the 4-row grouping of the sample row covers).
     ca.halo = halo_class(radius);
-    if ((rc = launch_check(ca, ring ? radius : 0, nt, s))) return rc;
+    if ((rc = launch_check(ca, ring_check, nt, s))) return rc;
     // exact fallback over the listed tiles
-    if (ring) return ring64_tiles(job, radius, mode, ws.list, ws.count, nt, s);
+    if (ring) return launch_ring(rjob, 0, nt, ws.list, ws.count, s);
     return exact_tiles(job, ws.list, nt, ws.count, 0, halo_class(radius), s);
 }
 
