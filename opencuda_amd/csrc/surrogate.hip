@@ -533,11 +533,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) w
     static_assert(KIND == K_HIDDEN || KIND == K_LAST, "32-channel inputs only");
     constexpr int CIN = C;
     constexpr int COUT = (KIND == K_LAST) ? 1 : C;
-    constexpr int M = 9 * CIN;
-    constexpr int MT = M / 16;                    // one tap per M-tile
     constexpr int NT = (COUT + 15) / 16;
-    constexpr int PAIRS = MT * NT;
-    constexpr int PPW = (PAIRS + 3) / 4;
+    // A wave's output tiles: one half of the input channels (16 rows per tap)
+    // and, hidden, one half of the outputs for all nine taps; last (one
+    // output), taps 0..4 (waves 0, 1) or 5..8.
+    constexpr int PPW = (KIND == K_LAST) ? 5 : 9;
     constexpr int PSZ = 9 * CIN * COUT + COUT;
     constexpr int DROWS = NT * 16;
     __shared__ __align__(16) __bf16 s_in[3][CIN][WG_PITCH];
@@ -546,6 +546,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) w
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i16 = lane & 15, kq = lane >> 4;
+    const int wcih = wave & 1, wnt = (KIND == K_LAST) ? 0 : wave >> 1;
+    const int wt0 = (KIND == K_LAST) ? PPW * (wave >> 1) : 0;      // first tap
     const int segs_x = (a.W + TX - 1) / TX;
     const int64_t nseg = (int64_t)a.N * a.H * segs_x;
     const int64_t npix = (int64_t)a.H * a.W;
@@ -642,30 +644,37 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) w
         __syncthreads();
         // the next segment's loads are in flight during this segment's MFMAs
         if (seg + gridDim.x < nseg) load_seg(seg + gridDim.x);
+        // Shifting the gradient instead of the input leaves the A operand of a
+        // tap independent of dx, and B of dy: a wave's taps share the rows'
+        // three A and the copies' three B operands of each K step.
 #pragma unroll
-        for (int q = 0; q < PPW; q++) {
-            const int pair = wave * PPW + q;
-            if (pair >= PAIRS) break;
-            const int mt = pair / NT, nt = pair - mt * NT;
-            const int t = (16 * mt) / CIN, ci = (16 * mt) % CIN + i16;
-            const int dy = t / 3 - 1, dx = t % 3 - 1;
+        for (int ks = 0; ks < TX / 32; ks++) {
+            bf16x8 av[3], bv[3];
 #pragma unroll
-            for (int ks = 0; ks < TX / 32; ks++) {
-                const bf16x8 av = *reinterpret_cast<const bf16x8 *>(&s_in[dy + 1][ci][32 * ks + 8 * kq]);
-                const bf16x8 bv = *reinterpret_cast<const bf16x8 *>(&s_d[dx + 1][16 * nt + i16][32 * ks + 8 * kq]);
-                acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[q], 0, 0, 0);
+            for (int d = 0; d < 3; d++) {
+                av[d] = *reinterpret_cast<const bf16x8 *>(&s_in[d][16 * wcih + i16][32 * ks + 8 * kq]);
+                bv[d] = *reinterpret_cast<const bf16x8 *>(&s_d[d][16 * wnt + i16][32 * ks + 8 * kq]);
+            }
+#pragma unroll
+            for (int q = 0; q < PPW; q++) {
+                if (KIND == K_HIDDEN) {
+                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[q / 3], bv[q % 3], acc[q], 0, 0, 0);
+                } else if (wave < 2) {
+                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[q / 3], bv[q % 3], acc[q], 0, 0, 0);
+                } else if (q + PPW < 9) {
+                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[(q + PPW) / 3], bv[(q + PPW) % 3], acc[q], 0, 0, 0);
+                }
             }
         }
     }
     float *part = a.partial + (size_t)blockIdx.x * PSZ;
 #pragma unroll
     for (int q = 0; q < PPW; q++) {
-        const int pair = wave * PPW + q;
-        if (pair >= PAIRS) break;
-        const int mt = pair / NT, nt = pair - mt * NT;
+        const int t = wt0 + q;
+        if (t >= 9) break;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int m = 16 * mt + 4 * kq + r, co = 16 * nt + i16;
+            const int m = t * CIN + 16 * wcih + 4 * kq + r, co = 16 * wnt + i16;
             if (co < COUT) part[m * COUT + co] = acc[q][r];
         }
     }
