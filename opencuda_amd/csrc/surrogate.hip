@@ -518,15 +518,21 @@ __device__ __forceinline__ void transpose8x8(const uint4 (&v)[8], uint4 (&out)[8
 // Weight gradients of the 32-input-channel layers (hidden, last), same
 // result layout as wgrad_kernel.  The column shift of a tap is moved onto the
 // gradient: sum_x in[y+dy][x+dx] d[y][x] = sum_x' in[y+dy][x'] d[y][x'-dx],
-// with both factors zero outside the crop, so a segment of 64 input columns
-// x' needs its three input rows without a column halo and three copies of
-// the one gradient row shifted by dx = -1, 0, 1.  Both are transposed in
-// registers (8 pixels x 8 channels per thread) and written to LDS as 16-byte
-// rows, K = pixels contiguous for the MFMA operands.
+// with both factors zero outside the crop, so a row of 64 input columns x'
+// needs three input rows without a column halo and three copies of the one
+// gradient row shifted by dx = -1, 0, 1.  Both are transposed in registers
+// (8 pixels x 8 channels per lane) and written to LDS as 16-byte rows, K =
+// pixels contiguous for the MFMA operands.
+//
+// A workgroup walks runs of rows down 64-column strips: each step adds one
+// input row (wave 0) and one gradient row (waves 1..3, one shifted copy each)
+// to rings in LDS, loaded into registers a step ahead, while the MFMAs run on
+// the rows already there; one barrier a step.  (Bound by memory and the
+// staging beside it.  Hidden layer on 64 crops of 256 x 256: 177 us; staging
+// three input rows per segment of a grid-wide order, with two barriers, 278.)
 constexpr int WG_PITCH = TX + 8;   // LDS row of 64 pixels + 8 pad (bank spread)
 
-// Register budget for 3 waves per SIMD (3 resident workgroups per CU; with
-// no bound the compiler's operand prefetch left 2, a budget for 4 spills).
+// Register budget for 3 waves per SIMD (3 resident workgroups per CU).
 template <int KIND>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) wgrad32_kernel(WgradArgs a)
 {
@@ -540,129 +546,129 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) w
     constexpr int PPW = (KIND == K_LAST) ? 5 : 9;
     constexpr int PSZ = 9 * CIN * COUT + COUT;
     constexpr int DROWS = NT * 16;
-    __shared__ __align__(16) __bf16 s_in[3][CIN][WG_PITCH];
-    __shared__ __align__(16) __bf16 s_d[3][DROWS][WG_PITCH];
+    __shared__ __align__(16) __bf16 s_in[4][CIN][WG_PITCH];        // input row r in slot r & 3
+    __shared__ __align__(16) __bf16 s_d[2][3][DROWS][WG_PITCH];    // gradient row y in slot y & 1
     __shared__ float s_bias[64];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i16 = lane & 15, kq = lane >> 4;
     const int wcih = wave & 1, wnt = (KIND == K_LAST) ? 0 : wave >> 1;
     const int wt0 = (KIND == K_LAST) ? PPW * (wave >> 1) : 0;      // first tap
     const int segs_x = (a.W + TX - 1) / TX;
-    const int64_t nseg = (int64_t)a.N * a.H * segs_x;
     const int64_t npix = (int64_t)a.H * a.W;
 
-    // Staging tasks.  Threads 0..95: input row r = y-1+(tid>>5), channel
-    // chunk (tid>>3)&3, pixels 8*(tid&7)..+7.  Hidden, threads 96..191:
-    // gradient copy dxi = (u>>5), same chunk/pixel split.  Last layer,
-    // threads 0..191: one pixel of one gradient copy (dxi = tid / 64).
-    const bool in_task = tid < 96;
-    const bool d_task = (KIND == K_HIDDEN) ? (tid >= 96 && tid < 192) : (tid < 192);
-    const int u = (KIND == K_HIDDEN) ? tid - 96 : tid;
-    const int t_row = tid >> 5, t_chunk = (tid >> 3) & 3, t_xg = tid & 7;
-    const int d_dxi = (KIND == K_HIDDEN) ? (u >> 5) : (u >> 6);
-    const int d_chunk = (u >> 3) & 3, d_xg = u & 7, d_xx = u & 63;
-
-    uint4 v[8];   // the thread's 8 pixels x 8 channels (input or gradient task)
+    // Staging: wave 0 the input row, wave 1 + dxi the gradient copy shifted by
+    // dxi - 1.  32-channel rows: lanes 0..31, channel chunk lane / 8, pixels
+    // 8 (lane % 8) .. + 7.  Last layer's gradient: one pixel a lane.
+    const bool wide = wave == 0 || KIND == K_HIDDEN;
+    const bool task = wide ? lane < 32 : true;
+    const int chunk = (lane >> 3) & 3, xg = lane & 7, dxi = wave - 1;
+    uint4 v[8];
     __bf16 vd1 = to_bf(0.0f);
-    auto load_seg = [&](int64_t seg) {
-        const int n = (int)(seg / ((int64_t)a.H * segs_x));
-        const int rem = (int)(seg - (int64_t)n * a.H * segs_x);
-        const int y = rem / segs_x, x0 = (rem - y * segs_x) * TX;
-        if (in_task) {
-            const int gy = y - 1 + t_row;
+    // item y of a column (crop n, strip x0): input row y + 1, gradient row y
+    auto load = [&](int n, int x0, int y) {
+        if (wide) {
+            const int row = wave == 0 ? y + 1 : y, shift = wave == 0 ? 0 : dxi - 1;
+            const __bf16 *src = (wave == 0 ? a.act : a.dpre) + ((size_t)n * npix + (size_t)max(row, 0) * a.W) * C + chunk * 8;
+            if (task) {
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int gx = x0 + 8 * t_xg + j;
-                v[j] = make_uint4(0, 0, 0, 0);
-                if (gy >= 0 && gy < a.H && gx < a.W)
-                    v[j] = *reinterpret_cast<const uint4 *>(a.act + ((size_t)n * npix + (size_t)gy * a.W + gx) * C + t_chunk * 8);
+                for (int j = 0; j < 8; j++) {
+                    const int gx = x0 + 8 * xg + j - shift;
+                    v[j] = make_uint4(0, 0, 0, 0);
+                    if (row >= 0 && row < a.H && gx >= 0 && gx < a.W)
+                        v[j] = *reinterpret_cast<const uint4 *>(src + (size_t)gx * C);
+                }
             }
-        }
-        if (KIND == K_HIDDEN && d_task) {
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int gx = x0 + 8 * d_xg + j - (d_dxi - 1);
-                v[j] = make_uint4(0, 0, 0, 0);
-                if (gx >= 0 && gx < a.W)
-                    v[j] = *reinterpret_cast<const uint4 *>(a.dpre + ((size_t)n * npix + (size_t)y * a.W + gx) * C + d_chunk * 8);
-            }
-        }
-        if (KIND == K_LAST && d_task) {
-            const int gx = x0 + d_xx - (d_dxi - 1);
+        } else {
+            const int gx = x0 + lane - (dxi - 1);
             vd1 = to_bf(0.0f);
             if (gx >= 0 && gx < a.W) vd1 = a.dpre[(size_t)n * npix + (size_t)y * a.W + gx];
         }
     };
+    // bias gradient, accumulated by the unshifted copy's wave: hidden, 8
+    // channels of 8 pixels per lane; last, one pixel per lane
+    float bsum[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
+    auto store = [&](int y) {
+        if (wide) {
+            if (task) {
+                uint4 t[8];
+                transpose8x8(v, t);
+                __bf16 *dst = wave == 0 ? &s_in[(y + 1) & 3][chunk * 8][8 * xg] : &s_d[y & 1][dxi][chunk * 8 % DROWS][8 * xg];
+#pragma unroll
+                for (int q = 0; q < 8; q++) *reinterpret_cast<uint4 *>(dst + q * WG_PITCH) = t[q];
+                if (dxi == 1) {
+#pragma unroll
+                    for (int q = 0; q < 8; q++) {
+                        const uint32_t *w = reinterpret_cast<const uint32_t *>(&t[q]);
+                        float sq = 0.0f;
+#pragma unroll
+                        for (int k = 0; k < 4; k++)
+                            sq += __uint_as_float(w[k] << 16) + __uint_as_float(w[k] & 0xFFFF0000u);
+                        bsum[q] += sq;
+                    }
+                }
+            }
+        } else {
+            s_d[y & 1][dxi][0][lane] = vd1;
+            if (dxi == 1) bsum[0] += from_bf(vd1);
+        }
+    };
 
     if (KIND == K_LAST) {   // gradient rows 1..15 of the single output channel stay zero
-        for (int e = tid; e < 3 * 15 * TX; e += 256) {
-            const int dxi = e / (15 * TX), rem = e - dxi * 15 * TX;
-            s_d[dxi][1 + rem / TX][rem % TX] = to_bf(0.0f);
+        for (int e = tid; e < 6 * 15 * TX; e += 256) {
+            const int c = e / (15 * TX), rem = e - c * 15 * TX;
+            s_d[c / 3][c % 3][1 + rem / TX][rem % TX] = to_bf(0.0f);
         }
     }
 
     f32x4 acc[PPW];
 #pragma unroll
     for (int q = 0; q < PPW; q++) acc[q] = (f32x4){ 0.f, 0.f, 0.f, 0.f };
-    // bias gradient, accumulated by the unshifted gradient copy's tasks:
-    // hidden, 8 channels of 8 pixels per thread; last, one pixel per thread
-    float bsum[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
 
-    if ((int64_t)blockIdx.x < nseg) load_seg(blockIdx.x);
-    for (int64_t seg = blockIdx.x; seg < nseg; seg += gridDim.x) {
-        __syncthreads();   // the previous segment's MFMAs are done with the LDS rows
-        if (in_task) {
-            uint4 t[8];
-            transpose8x8(v, t);
-#pragma unroll
-            for (int q = 0; q < 8; q++)
-                *reinterpret_cast<uint4 *>(&s_in[t_row][t_chunk * 8 + q][8 * t_xg]) = t[q];
+    // this workgroup's rows of all columns, in (crop, strip, row) order
+    const int64_t rows = (int64_t)a.N * segs_x * a.H;
+    int64_t cur = rows * blockIdx.x / gridDim.x;
+    const int64_t end = rows * (blockIdx.x + 1) / gridDim.x;
+    while (cur < end) {
+        const int64_t colm = cur / a.H;
+        const int ya = (int)(cur - colm * a.H);
+        const int yb = (int)min((int64_t)a.H, ya + (end - cur));
+        const int n = (int)(colm / segs_x), x0 = (int)(colm - (int64_t)n * segs_x) * TX;
+        cur += yb - ya;
+        __syncthreads();                          // the previous run's MFMAs are done
+        if (wave == 0) {                          // rows ya - 1 and ya
+            load(n, x0, ya - 2);
+            store(ya - 2);
+            load(n, x0, ya - 1);
+            store(ya - 1);
         }
-        if (KIND == K_HIDDEN && d_task) {
-            uint4 t[8];
-            transpose8x8(v, t);
+        load(n, x0, ya);
+        store(ya);
+        if (ya + 1 < yb) load(n, x0, ya + 1);
+        for (int y = ya; y < yb; y++) {
+            __syncthreads();                      // row y's items are in; row y - 1's MFMAs are done
+            if (y + 1 < yb) {
+                store(y + 1);
+                if (y + 2 < yb) load(n, x0, y + 2);
+            }
+            // Shifting the gradient instead of the input leaves the A operand
+            // of a tap independent of dx, and B of dy: a wave's taps share the
+            // rows' three A and the copies' three B operands of each K step.
 #pragma unroll
-            for (int q = 0; q < 8; q++)
-                *reinterpret_cast<uint4 *>(&s_d[d_dxi][d_chunk * 8 + q][8 * d_xg]) = t[q];
-            if (d_dxi == 1) {
+            for (int ks = 0; ks < TX / 32; ks++) {
+                bf16x8 av[3], bv[3];
 #pragma unroll
-                for (int q = 0; q < 8; q++) {
-                    const uint32_t *w = reinterpret_cast<const uint32_t *>(&t[q]);
-                    float sq = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < 4; k++)
-                        sq += __uint_as_float(w[k] << 16) + __uint_as_float(w[k] & 0xFFFF0000u);
-                    bsum[q] += sq;
+                for (int d = 0; d < 3; d++) {
+                    av[d] = *reinterpret_cast<const bf16x8 *>(&s_in[(y - 1 + d) & 3][16 * wcih + i16][32 * ks + 8 * kq]);
+                    bv[d] = *reinterpret_cast<const bf16x8 *>(&s_d[y & 1][d][16 * wnt + i16][32 * ks + 8 * kq]);
                 }
-            }
-        }
-        if (KIND == K_LAST && d_task) {
-            s_d[d_dxi][0][d_xx] = vd1;
-            if (d_dxi == 1) bsum[0] += from_bf(vd1);
-        }
-        __syncthreads();
-        // the next segment's loads are in flight during this segment's MFMAs
-        if (seg + gridDim.x < nseg) load_seg(seg + gridDim.x);
-        // Shifting the gradient instead of the input leaves the A operand of a
-        // tap independent of dx, and B of dy: a wave's taps share the rows'
-        // three A and the copies' three B operands of each K step.
 #pragma unroll
-        for (int ks = 0; ks < TX / 32; ks++) {
-            bf16x8 av[3], bv[3];
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                av[d] = *reinterpret_cast<const bf16x8 *>(&s_in[d][16 * wcih + i16][32 * ks + 8 * kq]);
-                bv[d] = *reinterpret_cast<const bf16x8 *>(&s_d[d][16 * wnt + i16][32 * ks + 8 * kq]);
-            }
-#pragma unroll
-            for (int q = 0; q < PPW; q++) {
-                if (KIND == K_HIDDEN) {
-                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[q / 3], bv[q % 3], acc[q], 0, 0, 0);
-                } else if (wave < 2) {
-                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[q / 3], bv[q % 3], acc[q], 0, 0, 0);
-                } else if (q + PPW < 9) {
-                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[(q + PPW) / 3], bv[(q + PPW) % 3], acc[q], 0, 0, 0);
+                for (int q = 0; q < PPW; q++) {
+                    if (KIND == K_HIDDEN || wave < 2)
+                        acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[q / 3], bv[q % 3], acc[q], 0, 0, 0);
+                    else if (q + PPW < 9)
+                        acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[(q + PPW) / 3], bv[(q + PPW) % 3], acc[q], 0, 0, 0);
                 }
             }
         }
@@ -678,24 +684,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) w
             if (co < COUT) part[m * COUT + co] = acc[q][r];
         }
     }
-    // bias: sum the unshifted copy's per-thread sums in a fixed order
+    // bias: sum the unshifted copy's per-lane sums in a fixed order
+    const bool btask = task && dxi == 1;
     if (KIND == K_HIDDEN) {
-        if (d_task && d_dxi == 1) {
+        if (btask && xg == 0) {
 #pragma unroll
-            for (int q = 0; q < 8; q++)
-                if (d_xg == 0) s_bias[d_chunk * 8 + q] = 0.0f;
+            for (int q = 0; q < 8; q++) s_bias[chunk * 8 + q] = 0.0f;
         }
         __syncthreads();
-        for (int xg = 0; xg < 8; xg++) {
-            if (d_task && d_dxi == 1 && d_xg == xg) {
+        for (int g = 0; g < 8; g++) {
+            if (btask && xg == g) {
 #pragma unroll
-                for (int q = 0; q < 8; q++) s_bias[d_chunk * 8 + q] += bsum[q];
+                for (int q = 0; q < 8; q++) s_bias[chunk * 8 + q] += bsum[q];
             }
             __syncthreads();
         }
         if (tid < COUT) part[9 * CIN * COUT + tid] = s_bias[tid];
     } else {
-        if (d_task && d_dxi == 1) s_bias[d_xx] = bsum[0];
+        if (btask) s_bias[lane] = bsum[0];
         __syncthreads();
         if (tid == 0) {
             float b = 0.0f;
