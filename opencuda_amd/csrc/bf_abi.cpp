@@ -12,6 +12,7 @@
 #include <string>
 #include <thread>
 #include <unordered_map>
+#include <utility>
 #include <vector>
 
 #include "bf_internal.h"
@@ -623,15 +624,19 @@ int bf_exact_inplace(const bf_image_view *img, bf_lut lut, int32_t radius, int32
     if (!tmp) BF_HIP(hipMallocAsync(reinterpret_cast<void **>(&tmp), bytes, s));
     bf_image_view scratch{ tmp, img->width, img->height, img->width };
     int rc = kOk;
-    // Each pass: snapshot the image into scratch, filter scratch -> image.
-    for (int i = 0; i < repeat && rc == kOk; i++) {
+    // Passes alternate between the image and the scratch (each reads what the
+    // one before wrote and nothing else); an odd count starts from a copy of
+    // the image in the scratch, so that the last pass ends in the image.
+    const bf_image_view *from = img, *to = &scratch;
+    if (repeat & 1) {
         hipError_t e = hipMemcpy2DAsync(tmp, img->width, img->data, img->pitch, img->width,
                                         img->height, hipMemcpyDeviceToDevice, s);
-        if (e != hipSuccess) {
-            rc = hip_fail(e, "hipMemcpy2DAsync");
-            break;
-        }
-        rc = bf_exact(&scratch, img, lut, radius, mode, stream);
+        if (e != hipSuccess) rc = hip_fail(e, "hipMemcpy2DAsync");
+        std::swap(from, to);
+    }
+    for (int i = 0; i < repeat && rc == kOk; i++) {
+        rc = bf_exact(from, to, lut, radius, mode, stream);
+        std::swap(from, to);
     }
     if (!work) {
         hipError_t e = hipFreeAsync(tmp, s);
