@@ -546,12 +546,18 @@ int launch_ring_check_one(const CheckArgs &a, int ntiles, hipStream_t s)
 
 }  // namespace
 
-// Tile config of a single image.  Both shapes hold the same lanes per SIMD
-// while two 64 x 32 workgroups fit a CU beside their tables (r <= 9).  Above,
-// a CU runs one workgroup, and a 64 x 32 tile takes about 0.6 of a 64 x 64
-// one's time (its two waves a SIMD cover less latency): it wins where halving
-// the tiles does not add rounds, on images of up to about 700^2 (640 x 480,
-// r = 14 REF: 75 against 125 us).
+// Tile config of a single image.
+// r <= 8: several workgroups share a CU, and the image takes as long as the
+// CU with the most waves; 64 x 16 tiles (four waves) spread them more evenly
+// than 64 x 32 ones (eight) on images of few tiles, and cost about 7% where
+// they do not, for their halo rows (r = 7 REF, us: 1021 x 767 25.6 against
+// 33.1, 1279 x 1024 41.1 against 45.6, 1600 x 1200 63.1 against 62.6, 2048^2
+// 115.7 against 107.6).
+// r = 9: 64 x 32 and 64 x 64 tiles hold the same lanes per SIMD.  Above, a CU
+// runs one workgroup, and a 64 x 32 tile takes about 0.6 of a 64 x 64 one's
+// time (its two waves a SIMD cover less latency): it wins where halving the
+// tiles does not add rounds, on images of up to about 700^2 (640 x 480,
+// r = 14 REF: 71 against 125 us).
 // REF from r = 17 forms many factors per tap here too, and below 12 Mpix the
 // tap list on 64 x 16 tiles, whose small table leaves room for several
 // workgroups a CU, fills the last round better (1500 x 1100, r = 18: 318
@@ -559,20 +565,25 @@ int launch_ring_check_one(const CheckArgs &a, int ntiles, hipStream_t s)
 // 2.32): -1.
 int ring_config(int radius, int mode, int W, int H)
 {
-    if (radius <= 9) return 1;
     if (mode == kModeRef && radius >= 17) return (int64_t)W * H < 12000000 ? -1 : 0;
+    if (radius == 9) return 1;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-        return 0;
-    const int64_t tx = (W + 63) / 64, t64 = tx * ((H + 63) / 64), t32 = tx * ((H + 31) / 32);
-    return 6 * ((t32 + cus - 1) / cus) < 10 * ((t64 + cus - 1) / cus) ? 1 : 0;
+        return radius <= 9 ? 1 : 0;
+    const int64_t tx = (W + 63) / 64;
+    auto rounds = [&](int th) { return (tx * ((H + th - 1) / th) + cus - 1) / cus; };   // tiles of the fullest CU
+    // r = 5, 6 stage the 8-pixel halo of r = 8 too: 64 x 16 tiles cost them more
+    const int more = radius == 5 || radius == 6 ? 125 : 107;
+    if (radius <= 8) return more * 4 * rounds(16) < 100 * 8 * rounds(32) ? 3 : 1;
+    return 6 * rounds(32) < 10 * rounds(64) ? 1 : 0;
 }
 
 // 64 x 64 tiles also serve tile lists (the surrogate's fallback) from r = 9.
 bool ring_kernel_available(int radius, int mode, int config)
 {
     if (radius < 1 || radius > BF_MAX_RADIUS) return false;
+    if (config == 3) return radius <= 8;
     return config == 0 ? radius >= 9 : (config == 1 && (mode != kModeRef || radius <= 16));
 }
 
@@ -601,6 +612,13 @@ int launch_ring(const DevJob &job, int config, int ntiles, const int32_t *list, 
         return kInvalidData;
     }
     const bool ref = job.mode == kModeRef;
+    if (config == 3) {
+        if (job.radius <= 4)
+            return ref ? launch_ring_one<0, 64, 4, 4>(job, ntiles, list, count, s)
+                       : launch_ring_one<1, 64, 4, 4>(job, ntiles, list, count, s);
+        return ref ? launch_ring_one<0, 64, 4, 8>(job, ntiles, list, count, s)
+                   : launch_ring_one<1, 64, 4, 8>(job, ntiles, list, count, s);
+    }
     if (config == 1) {
         switch (halo_class(job.radius)) {
         case 4: return ref ? launch_ring_one<0, 64, 8, 4>(job, ntiles, list, count, s)

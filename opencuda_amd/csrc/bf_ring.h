@@ -68,8 +68,11 @@ int launch_ring_one(const DevJob &job, int ntiles, const int32_t *list, const in
 #define BF_RING_KERNEL(X, MODE, TW, TGY, HALO)                                                 \
     X template int launch_ring_one<MODE, TW, TGY, HALO>(const DevJob &, int, const int32_t *, \
                                                         const int32_t *, hipStream_t);
-// The instances: 64 x 32 tiles (REF to r = 16), 64 x 64 tiles from r = 9.
+// The instances: 64 x 16 tiles to r = 8, 64 x 32 tiles (REF to r = 16), 64 x
+// 64 tiles from r = 9.
 #define BF_RING_SMALL(X, MODE)           \
+    BF_RING_KERNEL(X, MODE, 64, 4, 4)    \
+    BF_RING_KERNEL(X, MODE, 64, 4, 8)    \
     BF_RING_KERNEL(X, MODE, 64, 8, 4)    \
     BF_RING_KERNEL(X, MODE, 64, 8, 8)    \
     BF_RING_KERNEL(X, MODE, 64, 8, 12)
