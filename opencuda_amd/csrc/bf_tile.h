@@ -484,14 +484,28 @@ hipError_t allow_full_lds()
 }
 
 // Workgroups of `kern` (NT threads, lds bytes) that run at once on the
-// device; 0 when one does not fit.
+// device; 0 when one does not fit.  The answer depends on nothing else, so a
+// thread keeps its last few (the queries are most of a small launch's host
+// time).
 inline int resident_groups(const void *kern, int nt, size_t lds)
 {
+    struct Entry {
+        const void *kern;
+        size_t lds;
+        int nt, dev, groups;
+    };
+    constexpr int kEntries = 8;
+    thread_local Entry last[kEntries] = {};
+    thread_local int next = 0;
     int dev = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+    if (hipGetDevice(&dev) != hipSuccess) return -1;
+    for (const Entry &e : last)
+        if (e.kern == kern && e.lds == lds && e.nt == nt && e.dev == dev) return e.groups;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, nt, lds) != hipSuccess)
         return -1;
+    last[next] = Entry{ kern, lds, nt, dev, cus * per_cu };
+    next = (next + 1) % kEntries;
     return cus * per_cu;
 }
 
