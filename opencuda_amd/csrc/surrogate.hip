@@ -524,12 +524,13 @@ __device__ __forceinline__ void transpose8x8(const uint4 (&v)[8], uint4 (&out)[8
 // (8 pixels x 8 channels per lane) and written to LDS as 16-byte rows, K =
 // pixels contiguous for the MFMA operands.
 //
-// A workgroup walks runs of rows down 64-column strips: each step adds one
-// input row (wave 0) and one gradient row (waves 1..3, one shifted copy each)
-// to rings in LDS, loaded into registers a step ahead, while the MFMAs run on
-// the rows already there; one barrier a step.  (Bound by memory and the
-// staging beside it.  Hidden layer on 64 crops of 256 x 256: 177 us; staging
-// three input rows per segment of a grid-wide order, with two barriers, 278.)
+// A workgroup walks runs of rows down 64-column strips, two rows a step: each
+// step adds two input rows (wave 0) and two gradient rows (waves 1..3, one
+// shifted copy each) to rings in LDS, half a wave a row, loaded into
+// registers during the step before.  (Bound by memory and the staging beside
+// it.  64 crops of 256 x 256, hidden and last layer: 141 and 104 us; one row a
+// step, half of the lanes idle and half the bytes in flight, 177 and 152;
+// three input rows for every row in a grid-wide order 278 and 155.)
 constexpr int WG_PITCH = TX + 8;   // LDS row of 64 pixels + 8 pad (bank spread)
 
 // Register budget for 3 waves per SIMD (3 resident workgroups per CU).
@@ -558,60 +559,65 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) w
     const int segs_x = (a.W + TX - 1) / TX;
     const int64_t npix = (int64_t)a.H * a.W;
 
-    // Staging: wave 0 the input row, wave 1 + dxi the gradient copy shifted by
-    // dxi - 1.  32-channel rows: lanes 0..31, channel chunk lane / 8, pixels
-    // 8 (lane % 8) .. + 7.  Last layer's gradient: one pixel a lane.
+    // Staging: wave 0 the input rows, wave 1 + dxi the gradient copy shifted
+    // by dxi - 1.  32-channel rows: a row each for lanes 0..31 and 32..63,
+    // channel chunk (lane / 8) % 4, pixels 8 (lane % 8) .. + 7.  Last layer's
+    // gradient: one pixel of both rows a lane.
     const bool wide = wave == 0 || KIND == K_HIDDEN;
-    const bool task = wide ? lane < 32 : true;
-    const int chunk = (lane >> 3) & 3, xg = lane & 7, dxi = wave - 1;
+    const int half = lane >> 5, chunk = (lane >> 3) & 3, xg = lane & 7, dxi = wave - 1;
     uint4 v[8];
-    __bf16 vd1 = to_bf(0.0f);
-    // item y of a column (crop n, strip x0): input row y + 1, gradient row y
-    auto load = [&](int n, int x0, int y) {
+    __bf16 vd[2] = { to_bf(0.0f), to_bf(0.0f) };
+    // items y and y + 1 of a column (crop n, strip x0), where item y is input
+    // row y + 1 and gradient row y; gradient rows from y1 on are zero
+    auto load = [&](int n, int x0, int y, int y1) {
         if (wide) {
-            const int row = wave == 0 ? y + 1 : y, shift = wave == 0 ? 0 : dxi - 1;
+            const int row = y + half + (wave == 0 ? 1 : 0), shift = wave == 0 ? 0 : dxi - 1;
+            const int rows = wave == 0 ? a.H : y1;
             const __bf16 *src = (wave == 0 ? a.act : a.dpre) + ((size_t)n * npix + (size_t)max(row, 0) * a.W) * C + chunk * 8;
-            if (task) {
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int gx = x0 + 8 * xg + j - shift;
-                    v[j] = make_uint4(0, 0, 0, 0);
-                    if (row >= 0 && row < a.H && gx >= 0 && gx < a.W)
-                        v[j] = *reinterpret_cast<const uint4 *>(src + (size_t)gx * C);
-                }
+            for (int j = 0; j < 8; j++) {
+                const int gx = x0 + 8 * xg + j - shift;
+                v[j] = make_uint4(0, 0, 0, 0);
+                if (row >= 0 && row < rows && gx >= 0 && gx < a.W)
+                    v[j] = *reinterpret_cast<const uint4 *>(src + (size_t)gx * C);
             }
         } else {
             const int gx = x0 + lane - (dxi - 1);
-            vd1 = to_bf(0.0f);
-            if (gx >= 0 && gx < a.W) vd1 = a.dpre[(size_t)n * npix + (size_t)y * a.W + gx];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                vd[k] = to_bf(0.0f);
+                if (y + k < y1 && gx >= 0 && gx < a.W) vd[k] = a.dpre[(size_t)n * npix + (size_t)(y + k) * a.W + gx];
+            }
         }
     };
     // bias gradient, accumulated by the unshifted copy's wave: hidden, 8
-    // channels of 8 pixels per lane; last, one pixel per lane
+    // channels of 8 pixels per lane; last, one pixel column per lane
     float bsum[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
     auto store = [&](int y) {
         if (wide) {
-            if (task) {
-                uint4 t[8];
-                transpose8x8(v, t);
-                __bf16 *dst = wave == 0 ? &s_in[(y + 1) & 3][chunk * 8][8 * xg] : &s_d[y & 1][dxi][chunk * 8 % DROWS][8 * xg];
+            const int yy = y + half;
+            uint4 t[8];
+            transpose8x8(v, t);
+            __bf16 *dst = wave == 0 ? &s_in[(yy + 1) & 3][chunk * 8][8 * xg] : &s_d[yy & 1][dxi][chunk * 8 % DROWS][8 * xg];
 #pragma unroll
-                for (int q = 0; q < 8; q++) *reinterpret_cast<uint4 *>(dst + q * WG_PITCH) = t[q];
-                if (dxi == 1) {
+            for (int q = 0; q < 8; q++) *reinterpret_cast<uint4 *>(dst + q * WG_PITCH) = t[q];
+            if (dxi == 1) {
 #pragma unroll
-                    for (int q = 0; q < 8; q++) {
-                        const uint32_t *w = reinterpret_cast<const uint32_t *>(&t[q]);
-                        float sq = 0.0f;
+                for (int q = 0; q < 8; q++) {
+                    const uint32_t *w = reinterpret_cast<const uint32_t *>(&t[q]);
+                    float sq = 0.0f;
 #pragma unroll
-                        for (int k = 0; k < 4; k++)
-                            sq += __uint_as_float(w[k] << 16) + __uint_as_float(w[k] & 0xFFFF0000u);
-                        bsum[q] += sq;
-                    }
+                    for (int k = 0; k < 4; k++)
+                        sq += __uint_as_float(w[k] << 16) + __uint_as_float(w[k] & 0xFFFF0000u);
+                    bsum[q] += sq;
                 }
             }
         } else {
-            s_d[y & 1][dxi][0][lane] = vd1;
-            if (dxi == 1) bsum[0] += from_bf(vd1);
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                s_d[(y + k) & 1][dxi][0][lane] = vd[k];
+                if (dxi == 1) bsum[0] += from_bf(vd[k]);
+            }
         }
     };
 
@@ -637,20 +643,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) w
         const int n = (int)(colm / segs_x), x0 = (int)(colm - (int64_t)n * segs_x) * TX;
         cur += yb - ya;
         __syncthreads();                          // the previous run's MFMAs are done
-        if (wave == 0) {                          // rows ya - 1 and ya
-            load(n, x0, ya - 2);
+        if (wave == 0) {                          // input rows ya - 1 and ya
+            load(n, x0, ya - 2, yb);
             store(ya - 2);
-            load(n, x0, ya - 1);
-            store(ya - 1);
         }
-        load(n, x0, ya);
-        store(ya);
-        if (ya + 1 < yb) load(n, x0, ya + 1);
+        load(n, x0, ya, yb);
         for (int y = ya; y < yb; y++) {
-            __syncthreads();                      // row y's items are in; row y - 1's MFMAs are done
-            if (y + 1 < yb) {
-                store(y + 1);
-                if (y + 2 < yb) load(n, x0, y + 2);
+            if (((y - ya) & 1) == 0) {
+                __syncthreads();                  // the rows these replace are done with
+                store(y);
+                __syncthreads();
+                if (y + 2 < yb) load(n, x0, y + 2, yb);
             }
             // Shifting the gradient instead of the input leaves the A operand
             // of a tap independent of dx, and B of dy: a wave's taps share the
@@ -685,15 +688,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) w
         }
     }
     // bias: sum the unshifted copy's per-lane sums in a fixed order
-    const bool btask = task && dxi == 1;
+    const bool btask = dxi == 1;
     if (KIND == K_HIDDEN) {
-        if (btask && xg == 0) {
+        if (btask && xg == 0 && half == 0) {
 #pragma unroll
             for (int q = 0; q < 8; q++) s_bias[chunk * 8 + q] = 0.0f;
         }
         __syncthreads();
-        for (int g = 0; g < 8; g++) {
-            if (btask && xg == g) {
+        for (int g = 0; g < 16; g++) {
+            if (btask && 8 * half + xg == g) {
 #pragma unroll
                 for (int q = 0; q < 8; q++) s_bias[chunk * 8 + q] += bsum[q];
             }
