@@ -159,7 +159,8 @@ int bf_batch_unrolled(bf_batch batch);
  * sigma_space = radius/1.5, sigma_range = 30, run as a one-job batch with
  * that configuration (so the unrolled kernels are timed where a batch would
  * use them), `reps` timed launches after one warm-up -- and installs the
- * fastest in a process-wide table.  bf_exact and bf_batch_create (config < 0) use that
+ * fastest in a process-wide table.  bf_exact (where it runs the tap-list kernel) and
+ * bf_batch_create (config < 0) use that
  * table: a single image takes the tuned configuration of its radius; a
  * batch whose radii are all tuned takes the configuration with the least
  * estimated total time (sum over jobs of pixels x measured cost).
