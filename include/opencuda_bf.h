@@ -337,7 +337,8 @@ int bf_local_cluster(const bf_image_view *in, int64_t alloc_lo, int64_t alloc_hi
  * max_area], regions numbered in raster order of their first pixel, u8
  * output = number + 1 (0 = none).  Output size = min of the two views.
  * Allocates about 9.4 bytes per pixel of stream-ordered scratch (more per
- * pixel for images narrower than 64 columns).  Async. */
+ * pixel for images narrower than 64 columns).  Images of 2^26 rows and more,
+ * or of more than 2^31 - 1 pixels, are refused.  Async. */
 int bf_connect_region(const bf_image_view *in, const bf_image_view *out, int32_t min_area,
                       int32_t max_area, int32_t min_gray, int32_t max_gray, void *stream);
 

@@ -405,6 +405,7 @@ __device__ __forceinline__ bool cr_kept_area(const CrArgs &a, int ar)
 // does not count, is kept.
 constexpr int kCrT = 64;
 constexpr int kCrRuns = kCrT / 2;
+constexpr int kCrMaxRows = 1 << 26;     // rows are refused from here on (64 threads a row: 2^32)
 constexpr int kCrRow = kCrRuns + 1;      // run entries of a row in LDS (odd: rows fall in different banks)
 
 __device__ __forceinline__ int lds_load(const int *L, int i)
@@ -780,33 +781,33 @@ __global__ void __launch_bounds__(1024) cr_area_kernel(CrArgs a, int ntiles, int
     if (threadIdx.x < kCrSlots && key[threadIdx.x] >= 0) atomicAdd(a.area + key[threadIdx.x], sum_of[threadIdx.x]);
 }
 
-// One wave per row: which roots are kept, and how many.  The areas are read
-// here for the last time; from here on a.area holds the u8 numbers, 0 until
-// cr_number_kernel sets those of the first 256 kept roots.
+// One wave per row (of every 4 * gridDim.x): which roots are kept, and how
+// many.  The areas are read here for the last time; from here on a.area holds
+// the u8 numbers, 0 until cr_number_kernel sets those of the first 256 kept
+// roots.
 __global__ void __launch_bounds__(256) cr_kept_kernel(CrArgs a)
 {
     const int lane = (int)threadIdx.x & 63;
-    const int64_t y64 = (int64_t)blockIdx.x * 4 + ((int)threadIdx.x >> 6);
-    if (y64 >= a.H) return;                                      // whole waves
-    const int y = (int)y64;
-    int count = 0;
-    for (int tx = lane; tx < a.tiles_x; tx += 64) {
-        uint64_t bits = a.root[(int64_t)y * a.tiles_x + tx], kept = 0;
-        while (bits) {
-            const uint64_t bit = bits & (~bits + 1);
-            const int r = y * a.W + tx * kCrT + __ffsll((unsigned long long)bits) - 1;
-            bits ^= bit;
-            if (a.parent[r] == r) {
-                if (cr_kept_area(a, a.area[r])) kept |= bit;
-                a.area[r] = 0;
+    for (int y = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6); y < a.H; y += (int)gridDim.x * 4) {   // whole waves
+        int count = 0;
+        for (int tx = lane; tx < a.tiles_x; tx += 64) {
+            uint64_t bits = a.root[(int64_t)y * a.tiles_x + tx], kept = 0;
+            while (bits) {
+                const uint64_t bit = bits & (~bits + 1);
+                const int r = y * a.W + tx * kCrT + __ffsll((unsigned long long)bits) - 1;
+                bits ^= bit;
+                if (a.parent[r] == r) {
+                    if (cr_kept_area(a, a.area[r])) kept |= bit;
+                    a.area[r] = 0;
+                }
             }
+            a.kept[(int64_t)y * a.tiles_x + tx] = kept;
+            count += __popcll(kept);
         }
-        a.kept[(int64_t)y * a.tiles_x + tx] = kept;
-        count += __popcll(kept);
-    }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) count += __shfl_xor(count, off);
-    if (lane == 0) a.rowcount[y] = count;
+        for (int off = 32; off > 0; off >>= 1) count += __shfl_xor(count, off);
+        if (lane == 0) a.rowcount[y] = count;
+    }
 }
 
 // Raster-order numbers (one workgroup): kept roots before each row by a scan
@@ -1024,6 +1025,12 @@ int bf_connect_region(const bf_image_view *in, const bf_image_view *out, int32_t
         set_error("image too large for 32-bit labels");
         return kInvalidData;
     }
+    // A launch holds fewer than 2^32 threads in a dimension; the passes that
+    // follow a refused one would work on scratch it has not set.
+    if (H >= kCrMaxRows) {
+        set_error("image taller than 2^26 - 1 rows");
+        return kInvalidData;
+    }
     hipStream_t s = (hipStream_t)stream;
     const size_t n = (size_t)W * H;
     const int tiles_x = (W + kCrT - 1) / kCrT, tiles_y = (H + kCrT - 1) / kCrT;
@@ -1063,7 +1070,7 @@ int bf_connect_region(const bf_image_view *in, const bf_image_view *out, int32_t
     // four below, where the workgroups would not fill the device.
     const int per = ntiles >= 16 * 256 ? 2 : 1;
     hipLaunchKernelGGL(cr_area_kernel, dim3((ntiles + 4 * per - 1) / (4 * per)), dim3(1024), 0, s, a, ntiles, per);
-    hipLaunchKernelGGL(cr_kept_kernel, dim3((H + 3) / 4), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(cr_kept_kernel, dim3((unsigned)std::min((H + 3) / 4, 1 << 22)), dim3(256), 0, s, a);
     hipLaunchKernelGGL(cr_number_kernel, dim3(1), dim3(1024), 0, s, a);
     hipLaunchKernelGGL(cr_output_kernel, dim3(ntiles), dim3(256), 0, s, a);
     hipError_t e = hipGetLastError();
