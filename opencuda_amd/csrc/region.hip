@@ -1037,6 +1037,8 @@ int bf_connect_region(const bf_image_view *in, const bf_image_view *out, int32_t
         return kInvalidData;
     }
     hipStream_t s = (hipStream_t)stream;
+    int cus = 0;
+    BF_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, current_device()));
     const size_t n = (size_t)W * H;
     const int tiles_x = (W + kCrT - 1) / kCrT, tiles_y = (H + kCrT - 1) / kCrT;
     const int ntiles = tiles_x * tiles_y;
@@ -1070,10 +1072,12 @@ int bf_connect_region(const bf_image_view *in, const bf_image_view *out, int32_t
     a.run_root = reinterpret_cast<uint16_t *>(a.rowcount + H);
     hipLaunchKernelGGL(cr_local_kernel, dim3(ntiles), dim3(256), 0, s, a);
     hipLaunchKernelGGL(cr_union_kernel, dim3((unsigned)((2 * (int64_t)ntiles + 3) / 4)), dim3(256), 0, s, a, ntiles);
-    // Eight tiles a workgroup from 4,096 tiles on (fewer atomics on a region
-    // that spans the image: 18.8 us on a 4096 x 4096 image, 16 tiles 20.8),
-    // four below, where the workgroups would not fill the device.
-    const int per = ntiles >= 16 * 256 ? 2 : 1;
+    // Eight tiles a workgroup where that still gives every CU two, four below.
+    // Fewer workgroups add fewer sums to a region that spans the image; the
+    // whole call on square images, noise 2, four / eight tiles, in us: 65.6 /
+    // 70.1 at 2048, 92.5 / 92.4 at 3000, 122.0 / 121.6 at 3600, 122.5 / 119.2
+    // at 4096, 217 / 204 at 6000, 300 / 276 at 8192 (sixteen: 280).
+    const int per = ntiles >= 2 * 8 * cus ? 2 : 1;
     hipLaunchKernelGGL(cr_area_kernel, dim3((ntiles + 4 * per - 1) / (4 * per)), dim3(1024), 0, s, a, ntiles, per);
     hipLaunchKernelGGL(cr_kept_kernel, dim3((unsigned)std::min((H + 3) / 4, 1 << 22)), dim3(256), 0, s, a);
     hipLaunchKernelGGL(cr_number_kernel, dim3(1), dim3(1024), 0, s, a);
