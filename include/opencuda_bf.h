@@ -177,7 +177,13 @@ int bf_tune_get(int32_t radius, int32_t mode, float *ms_per_mpix);
 /* Forget every tuned entry (back to the built-in defaults). */
 int bf_tune_reset(void);
 
-/* bf_exact with an explicit tile configuration (the autotuner's probe). */
+/* What bf_exact runs on a width x height image: returns the tile
+ * configuration; *unrolled (may be NULL) receives 1 for an unrolled kernel of
+ * the canonical template, 0 for the tap-list kernel. */
+int bf_exact_plan(bf_lut lut, int32_t radius, int32_t mode, int32_t width, int32_t height,
+                  int32_t *unrolled);
+
+/* bf_exact on the tap-list kernel with an explicit tile configuration. */
 int bf_exact_config(const bf_image_view *in, const bf_image_view *out,
                     bf_lut lut, int32_t radius, int32_t mode, int32_t config,
                     void *stream);

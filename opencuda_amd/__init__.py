@@ -79,6 +79,7 @@ def lib() -> ctypes.CDLL:
         "bf_lut_rows": ([P, I32], ctypes.c_int),
         "bf_exact": ([VP, VP, P, I32, I32, P], ctypes.c_int),
         "bf_exact_config": ([VP, VP, P, I32, I32, I32, P], ctypes.c_int),
+        "bf_exact_plan": ([P, I32, I32, I32, I32, P], ctypes.c_int),
         "bf_exact_inplace": ([VP, P, I32, I32, I32, P, P], ctypes.c_int),
         "bf_tune_count": ([], ctypes.c_int),
         "bf_tune_describe": ([I32, P, P, P, P], ctypes.c_int),
@@ -231,6 +232,14 @@ def exact(vin: View, vout: View, lut: Lut, radius: int, mode: int = MODE_REF,
         rc = lib().bf_exact_config(ctypes.byref(vin), ctypes.byref(vout), lut.handle,
                                    int(radius), int(mode), int(config), s)
     _check(rc, "bf_exact")
+
+
+def exact_plan(lut: Lut, radius: int, mode: int, width: int, height: int):
+    """(tile config, unrolled) that bf_exact runs on a width x height image."""
+    u = ctypes.c_int32()
+    c = _check(lib().bf_exact_plan(lut.handle, int(radius), int(mode), int(width), int(height),
+                                   ctypes.byref(u)), "bf_exact_plan")
+    return c, bool(u.value)
 
 
 def exact_inplace(v: View, lut: Lut, radius: int, mode: int = MODE_REF, repeat: int = 1,

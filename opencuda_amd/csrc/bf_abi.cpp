@@ -468,6 +468,25 @@ int bf_exact_config(const bf_image_view *in, const bf_image_view *out, bf_lut lu
                         job.lut_rows, nullptr, (hipStream_t)stream);
 }
 
+// What bf_exact runs for a W x H image: an unrolled kernel on tiles of
+// `config` (ring) or the tap-list kernel.
+struct ExactPlan {
+    int config;
+    bool ring;
+};
+
+static ExactPlan plan_exact(const Lut *L, int radius, int mode, int W, int H)
+{
+    if (L->canonical && ring_rows(radius, mode) > 0 && ntaps_for(radius, mode) <= L->count) {
+        const int config = ring_config(radius, mode, W, H);
+        if (config >= 0) return { config, true };
+    }
+    const int rows = fused_rows(L, radius, mode);
+    const int tuned = tuned_config(radius, mode);
+    const int want = tuned >= 0 ? tuned : (radius >= 17 ? 3 : default_config(radius, mode));
+    return { rows < 0 ? default_config(1, mode) : fit_config(want, radius, rows), false };
+}
+
 int bf_exact(const bf_image_view *in, const bf_image_view *out, bf_lut lut, int32_t radius,
              int32_t mode, void *stream)
 {
@@ -475,30 +494,46 @@ int bf_exact(const bf_image_view *in, const bf_image_view *out, bf_lut lut, int3
         set_error("null lut");
         return kNullPointer;
     }
-    Lut *L = lut_from_handle(lut);
-    if (L->canonical && ring_rows(radius, mode) > 0 && ntaps_for(radius, mode) <= L->count) {
-        if (!in || !out) {
-            set_error("null argument");
-            return kNullPointer;
-        }
-        if (in->data && out->data && in->width > 0 && out->width > 0 && in->height > 0 &&
-            out->height > 0 && views_overlap(in, out)) {
-            set_error("input and output views overlap");
-            return kInvalidData;
-        }
-        const int rcfg = ring_config(radius, mode, std::min(in->width, out->width),
-                                     std::min(in->height, out->height));
-        DevJob job;
-        int rc = make_job(in, out, L, radius, mode, std::max(rcfg, 0), halo_class(radius), 0, &job, nullptr);
-        if (rc) return rc;
-        if (rcfg >= 0 && ring_job(L, radius, mode, rcfg, halo_class(radius), &job))
-            return launch_ring(job, rcfg, tiles_of(job, rcfg), nullptr, nullptr, (hipStream_t)stream);
+    if (!in || !out) {
+        set_error("null argument");
+        return kNullPointer;
     }
-    const int rows = fused_rows(lut_from_handle(lut), radius, mode);
-    const int tuned = tuned_config(radius, mode);
-    const int want = tuned >= 0 ? tuned : (radius >= 17 ? 3 : default_config(radius, mode));
-    const int config = rows < 0 ? default_config(1, mode) : fit_config(want, radius, rows);
-    return bf_exact_config(in, out, lut, radius, mode, config, stream);
+    Lut *L = lut_from_handle(lut);
+    const ExactPlan plan = plan_exact(L, radius, mode, std::min(in->width, out->width),
+                                      std::min(in->height, out->height));
+    if (!plan.ring) return bf_exact_config(in, out, lut, radius, mode, plan.config, stream);
+    if (in->data && out->data && in->width > 0 && out->width > 0 && in->height > 0 &&
+        out->height > 0 && views_overlap(in, out)) {
+        set_error("input and output views overlap");
+        return kInvalidData;
+    }
+    const int halo = halo_class(radius);
+    DevJob job;
+    int rc = make_job(in, out, L, radius, mode, plan.config, halo, 0, &job, nullptr);
+    if (rc) return rc;
+    if (!ring_job(L, radius, mode, plan.config, halo, &job)) {
+        set_error("template does not hold the unrolled kernel's taps");
+        return kInvalidData;
+    }
+    return launch_ring(job, plan.config, tiles_of(job, plan.config), nullptr, nullptr, (hipStream_t)stream);
+}
+
+int bf_exact_plan(bf_lut lut, int32_t radius, int32_t mode, int32_t width, int32_t height,
+                  int32_t *unrolled)
+{
+    if (!lut) {
+        set_error("null lut");
+        return kNullPointer;
+    }
+    Lut *L = lut_from_handle(lut);
+    if ((mode != BF_MODE_REF && mode != BF_MODE_STD) || width < 1 || height < 1 ||
+        fused_rows(L, radius, mode) < 0) {
+        set_error("bad radius, mode or size for this template");
+        return kInvalidData;
+    }
+    const ExactPlan plan = plan_exact(L, radius, mode, width, height);
+    if (unrolled) *unrolled = plan.ring ? 1 : 0;
+    return plan.config;
 }
 
 int bf_tune_radius(int32_t radius, int32_t mode, int32_t width, int32_t height, int32_t reps,
