@@ -575,7 +575,12 @@ int ring_config(int radius, int mode, int W, int H)
     auto rounds = [&](int th) { return (tx * ((H + th - 1) / th) + cus - 1) / cus; };   // tiles of the fullest CU
     // r = 5, 6 stage the 8-pixel halo of r = 8 too: 64 x 16 tiles cost them more
     const int more = radius == 5 || radius == 6 ? 125 : 107;
-    if (radius <= 8) return more * 4 * rounds(16) < 100 * 8 * rounds(32) ? 3 : 1;
+    // r = 8: the table leaves room for two 64 x 16 workgroups a CU, eight waves
+    // against sixteen, so they win only where each CU has one tile at most
+    // (us, 64 x 16 / 64 x 32, REF and STD: 512^2 25.1 / 26.6 and 24.1 / 26.8;
+    // 1021 x 767 46.7 / 41.6 and 47.7 / 47.1; 1700 x 1300 109 / 89 and 127 / 99)
+    if (radius == 8) return rounds(16) <= 1 ? 3 : 1;
+    if (radius < 8) return more * 4 * rounds(16) < 100 * 8 * rounds(32) ? 3 : 1;
     return 6 * rounds(32) < 10 * rounds(64) ? 1 : 0;
 }
 

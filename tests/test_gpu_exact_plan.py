@@ -73,6 +73,14 @@ def test_tap_list_below(device, r):
     _both(1101, 1099, r, REF, 3, unrolled=False)
 
 
+@pytest.mark.parametrize("mode", [REF, STD])
+@pytest.mark.parametrize("w,h,config", [(512, 512, 3), (1024, 256, 3), (513, 512, 1), (800, 800, 1),
+                                        (1021, 767, 1), (1700, 1300, 1)])
+def test_r8_tiles(device, w, h, config, mode):
+    # two 64 x 16 workgroups fit a CU: only images of one tile a CU take them
+    _both(w, h, 8, mode, config)
+
+
 def test_plan_refuses(device):
     lut = oc.Lut.from_sigmas(2.0, 20.0)
     for r, mode, w, h in ((0, REF, 9, 9), (21, STD, 9, 9), (20, REF, 9, 9), (3, 2, 9, 9), (3, REF, 0, 9)):
