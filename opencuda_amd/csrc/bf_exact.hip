@@ -573,8 +573,14 @@ int ring_config(int radius, int mode, int W, int H)
         return radius <= 9 ? 1 : 0;
     const int64_t tx = (W + 63) / 64;
     auto rounds = [&](int th) { return (tx * ((H + th - 1) / th) + cus - 1) / cus; };   // tiles of the fullest CU
-    // r = 5, 6 stage the 8-pixel halo of r = 8 too: 64 x 16 tiles cost them more
-    const int more = radius == 5 || radius == 6 ? 125 : 107;
+    // r = 5, 6 stage the 8-pixel halo of r = 8 too: 64 x 16 tiles cost them more.
+    // REF r = 7: three 64 x 16 workgroups a CU, twelve waves against 24; on
+    // quiet content, where the gathers meet few bank conflicts, they lose from
+    // seven tiles a CU on (us, 64 x 16 / 64 x 32, noise 10 and noise 1: 1279 x
+    // 1024, 5 and 3 tiles, 41.4 / 47.1 and 38.3 / 39.3; 1500 x 1150, 7 and 4,
+    // 57.3 / 57.5 and 54.3 / 47.3; 1700 x 1300, 9 and 5, 66.2 / 67.3 and 62.1
+    // / 55.0).
+    const int more = radius == 5 || radius == 6 ? 125 : (radius == 7 && mode == kModeRef ? 118 : 107);
     // r = 8: the table leaves room for two 64 x 16 workgroups a CU, eight waves
     // against sixteen, so they win only where each CU has one tile at most
     // (us, 64 x 16 / 64 x 32, REF and STD: 512^2 25.1 / 26.6 and 24.1 / 26.8;

@@ -81,6 +81,13 @@ def test_r8_tiles(device, w, h, config, mode):
     _both(w, h, 8, mode, config)
 
 
+@pytest.mark.parametrize("w,h,config", [(1021, 767, 3), (1279, 1024, 3), (1500, 1150, 1), (1700, 1300, 1),
+                                        (1900, 1400, 1)])
+def test_r7_ref_tiles(device, w, h, config):
+    # from seven 64 x 16 tiles a CU on, quiet images lose on them
+    _both(w, h, 7, REF, config)
+
+
 def test_plan_refuses(device):
     lut = oc.Lut.from_sigmas(2.0, 20.0)
     for r, mode, w, h in ((0, REF, 9, 9), (21, STD, 9, 9), (20, REF, 9, 9), (3, 2, 9, 9), (3, REF, 0, 9)):
