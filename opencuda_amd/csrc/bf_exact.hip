@@ -587,7 +587,11 @@ int ring_config(int radius, int mode, int W, int H)
     // 1021 x 767 46.7 / 41.6 and 47.7 / 47.1; 1700 x 1300 109 / 89 and 127 / 99)
     if (radius == 8) return rounds(16) <= 1 ? 3 : 1;
     if (radius < 8) return more * 4 * rounds(16) < 100 * 8 * rounds(32) ? 3 : 1;
-    return 6 * rounds(32) < 10 * rounds(64) ? 1 : 0;
+    // Above 9, in hundredths of a 64 x 64 round, a 64 x 32 round takes 56 to 71
+    // (REF), 60 to 73 (STD, r = 13 to 16, whose windows of 20 taps cover less
+    // of a gather's latency; noise 10 and filtered content).
+    const int part = mode != kModeRef && halo_class(radius) == 16 ? 67 : 60;
+    return part * rounds(32) < 100 * rounds(64) ? 1 : 0;
 }
 
 // 64 x 64 tiles also serve tile lists (the surrogate's fallback) from r = 9.

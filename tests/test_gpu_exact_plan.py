@@ -41,7 +41,7 @@ def test_64x16(device, r, w, h, mode):
 @pytest.mark.parametrize("r,w,h", [(1, 2047, 1535), (2, 2048, 1536), (3, 2047, 2049), (4, 2047, 1535),
                                    (5, 1601, 1203), (6, 1601, 1203), (7, 2048, 2047), (8, 2047, 1535),
                                    (9, 203, 139), (9, 1700, 1301), (10, 501, 499), (12, 1101, 1099),
-                                   (13, 700, 701), (16, 1100, 1101)])
+                                   (13, 700, 701), (16, 701, 700)])
 def test_64x32(device, r, w, h, mode):
     _both(w, h, r, mode, 1)
 
@@ -86,6 +86,13 @@ def test_r8_tiles(device, w, h, config, mode):
 def test_r7_ref_tiles(device, w, h, config):
     # from seven 64 x 16 tiles a CU on, quiet images lose on them
     _both(w, h, 7, REF, config)
+
+
+@pytest.mark.parametrize("r,mode,config", [(12, STD, 1), (13, STD, 0), (15, STD, 0), (16, STD, 0), (18, STD, 1),
+                                           (12, REF, 1), (13, REF, 1), (15, REF, 1), (16, REF, 1)])
+def test_three_rounds_against_two(device, r, mode, config):
+    # 1100 x 1100: three rounds of 64 x 32 tiles or two of 64 x 64
+    _both(1100, 1100, r, mode, config)
 
 
 def test_plan_refuses(device):
