@@ -546,26 +546,32 @@ int launch_ring_check_one(const CheckArgs &a, int ntiles, hipStream_t s)
 
 }  // namespace
 
-// Tile config of a single image.
+// Tile config of a single image.  Times in us on 256 CUs, noise 10 unless
+// said otherwise.
 // r <= 8: several workgroups share a CU, and the image takes as long as the
 // CU with the most waves; 64 x 16 tiles (four waves) spread them more evenly
 // than 64 x 32 ones (eight) on images of few tiles, and cost about 7% where
-// they do not, for their halo rows (r = 7 REF, us: 1021 x 767 25.6 against
-// 33.1, 1279 x 1024 41.1 against 45.6, 1600 x 1200 63.1 against 62.6, 2048^2
-// 115.7 against 107.6).
+// they do not, for their halo rows (r = 7 REF: 1021 x 767 25.6 against 33.1,
+// 1279 x 1024 41.1 against 45.6, 1600 x 1200 63.1 against 62.6, 2048^2 115.7
+// against 107.6; r = 4 REF: 1100 x 1000 16.5 against 18.2, 2048 x 1536 34.4
+// against 32.2).
 // r = 9: 64 x 32 and 64 x 64 tiles hold the same lanes per SIMD.  Above, a CU
 // runs one workgroup, and a 64 x 32 tile takes about 0.6 of a 64 x 64 one's
 // time (its two waves a SIMD cover less latency): it wins where halving the
-// tiles does not add rounds, on images of up to about 700^2 (640 x 480,
-// r = 14 REF: 71 against 125 us).
-// REF from r = 17 forms many factors per tap here too, and below 12 Mpix the
+// tiles adds few rounds, on images of one round of 64 x 32 tiles (r = 13 REF,
+// 700^2: 62 against 107, 1000^2, two against one: 116 against 108) and again
+// of three against two of 64 x 64 (1100^2 167 against 197, 1200^2 170 against
+// 198; 1300^2, four against two: 222 against 201).
+// REF from r = 17 forms many factors per tap here too, and below 10 Mpix the
 // tap list on 64 x 16 tiles, whose small table leaves room for several
-// workgroups a CU, fills the last round better (1500 x 1100, r = 18: 318
-// against 379 us; 3000^2, r = 17: 1.31 against 1.35 ms; 4096^2: 2.45 against
-// 2.32): -1.
+// workgroups a CU, fills the last round better: -1 (ms, tap list / unrolled,
+// r = 17, noise 10 and 1: 1500 x 1100 0.288 / 0.333 and 0.239 / 0.294; 2500^2
+// 0.95 / 1.05 and 0.86 / 0.88; 3000^2 1.31 / 1.35 and 1.18 / 1.18; 3300^2 1.61
+// / 1.61 and 1.48 / 1.37; 3800 x 3600 1.99 / 2.01 and 1.83 / 1.75; 4096^2, noise
+// 10, 2.44 / 2.30; 6000^2 5.28 / 4.81).
 int ring_config(int radius, int mode, int W, int H)
 {
-    if (mode == kModeRef && radius >= 17) return (int64_t)W * H < 12000000 ? -1 : 0;
+    if (mode == kModeRef && radius >= 17) return (int64_t)W * H < 10000000 ? -1 : 0;
     if (radius == 9) return 1;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -573,17 +579,21 @@ int ring_config(int radius, int mode, int W, int H)
         return radius <= 9 ? 1 : 0;
     const int64_t tx = (W + 63) / 64;
     auto rounds = [&](int th) { return (tx * ((H + th - 1) / th) + cus - 1) / cus; };   // tiles of the fullest CU
-    // r = 5, 6 stage the 8-pixel halo of r = 8 too: 64 x 16 tiles cost them more.
-    // REF r = 7: three 64 x 16 workgroups a CU, twelve waves against 24; on
-    // quiet content, where the gathers meet few bank conflicts, they lose from
-    // seven tiles a CU on (us, 64 x 16 / 64 x 32, noise 10 and noise 1: 1279 x
-    // 1024, 5 and 3 tiles, 41.4 / 47.1 and 38.3 / 39.3; 1500 x 1150, 7 and 4,
-    // 57.3 / 57.5 and 54.3 / 47.3; 1700 x 1300, 9 and 5, 66.2 / 67.3 and 62.1
-    // / 55.0).
-    const int more = radius == 5 || radius == 6 ? 125 : (radius == 7 && mode == kModeRef ? 118 : 107);
+    // REF r = 5, 6: four 64 x 16 workgroups a CU, 16 waves against 24 and 32;
+    // on quiet content, where the gathers meet few bank conflicts, they lose
+    // from five tiles a CU on (64 x 16 / 64 x 32, noise 10 and filtered: 1021
+    // x 767, three tiles, 15.9 / 19.0 and 14.8 / 16.3; 1279 x 1024, five, 24.7
+    // / 26.3 and 22.5 / 21.3; three passes in place there 83.7 / 81.6).  STD
+    // gains on all content (r = 5, 1279 x 1024: 24.0 / 27.0 and 22.0 / 23.3; 1700
+    // x 1300: 39.0 / 41.1 and 32.3 / 34.3).
+    // REF r = 7: three workgroups, twelve waves against 24; they lose from
+    // seven tiles a CU on (noise 10 and 1: 1279 x 1024, five, 41.4 / 47.1 and
+    // 38.3 / 39.3; 1500 x 1150, seven, 57.3 / 57.5 and 54.3 / 47.3; 1700 x 1300,
+    // nine, 66.2 / 67.3 and 62.1 / 55.0).
+    const int more = mode != kModeRef || radius <= 4 ? 107 : (radius == 7 ? 118 : 125);
     // r = 8: the table leaves room for two 64 x 16 workgroups a CU, eight waves
     // against sixteen, so they win only where each CU has one tile at most
-    // (us, 64 x 16 / 64 x 32, REF and STD: 512^2 25.1 / 26.6 and 24.1 / 26.8;
+    // (64 x 16 / 64 x 32, REF and STD: 512^2 25.1 / 26.6 and 24.1 / 26.8;
     // 1021 x 767 46.7 / 41.6 and 47.7 / 47.1; 1700 x 1300 109 / 89 and 127 / 99)
     if (radius == 8) return rounds(16) <= 1 ? 3 : 1;
     if (radius < 8) return more * 4 * rounds(16) < 100 * 8 * rounds(32) ? 3 : 1;

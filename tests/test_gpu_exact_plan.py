@@ -95,6 +95,19 @@ def test_three_rounds_against_two(device, r, mode, config):
     _both(1100, 1100, r, mode, config)
 
 
+@pytest.mark.parametrize("r", [5, 6])
+@pytest.mark.parametrize("w,h,mode,config", [(1021, 767, REF, 3), (1279, 1024, REF, 1), (1700, 1300, REF, 1),
+                                             (1279, 1024, STD, 3), (1700, 1300, STD, 3), (1600, 1200, STD, 1)])
+def test_r5_r6_tiles(device, r, w, h, mode, config):
+    _both(w, h, r, mode, config)
+
+
+@pytest.mark.parametrize("r", [17, 19])
+@pytest.mark.parametrize("w,h,unrolled", [(3001, 2999, False), (3300, 3300, True)])
+def test_ref_largest_radii_by_size(device, r, w, h, unrolled):
+    _both(w, h, r, REF, 0 if unrolled else 3, unrolled)
+
+
 def test_plan_refuses(device):
     lut = oc.Lut.from_sigmas(2.0, 20.0)
     for r, mode, w, h in ((0, REF, 9, 9), (21, STD, 9, 9), (20, REF, 9, 9), (3, 2, 9, 9), (3, REF, 0, 9)):
