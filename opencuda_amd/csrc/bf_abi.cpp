@@ -703,6 +703,18 @@ struct Batch {
 
 }  // namespace bfimpl
 
+// Every job on the canonical template and within its taps.
+static bool all_canonical(const bf_job *jobs, int njobs)
+{
+    for (int i = 0; i < njobs; i++) {
+        const Lut *L = lut_from_handle(jobs[i].lut);
+        if (!L || !L->canonical || ring_rows(jobs[i].radius, jobs[i].mode) <= 0 ||
+            ntaps_for(jobs[i].radius, jobs[i].mode) > L->count)
+            return false;
+    }
+    return true;
+}
+
 extern "C" {
 
 int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch *out)
@@ -726,6 +738,7 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
     // the least estimated time when every (radius, mode) is tuned, else the
     // built-in default for the largest radius.
     int cfg = config >= 0 ? config : default_config(rmax, jobs[0].mode);
+    bool tuned = false;
     if (config < 0) {
         TuneTable &t = tune_table();
         std::lock_guard<std::mutex> lock(t.mu);
@@ -749,6 +762,7 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
                 if (ok && (best < 0 || est < best)) {
                     best = est;
                     cfg = c;
+                    tuned = true;
                 }
             }
         }
@@ -781,7 +795,12 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
         cost[i] = (int64_t)dj[i].ntaps_padded;
         pixels += px;
     }
-    if (config < 0) {
+    // The unrolled kernels take what fits in LDS of a table beside any of their
+    // tiles, and costs of the canonical template were measured with its table
+    // as it runs beside a tile; only otherwise a configuration has to be found
+    // beside which the tables fit.
+    const bool canonical = all_canonical(jobs, njobs);
+    if (config < 0 && !(canonical && (tuned || ring_batch_supported(cfg, halo)))) {
         const int c = fit_config(cfg, rmax, max_rows);
         if (c != cfg) {   // re-plan the jobs with the configuration that fits
             cfg = c;
@@ -792,16 +811,14 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
             }
         }
     }
-    // Every job on the canonical template at a radius with an unrolled
-    // kernel: switch the whole batch to the per-q tables of those kernels.
-    bool ring = ring_batch_supported(cfg, halo);
-    if (ring) {
-        std::vector<DevJob> rj = dj;
-        for (int i = 0; i < njobs && ring; i++)
-            ring = ring_job(lut_from_handle(jobs[i].lut), jobs[i].radius, jobs[i].mode, cfg, halo,
-                            &rj[i]);
-        if (ring) dj.swap(rj);
-    }
+    // All on the canonical template, on tiles with unrolled kernels: those, with
+    // their per-q tables.
+    const bool ring = canonical && ring_batch_supported(cfg, halo);
+    for (int i = 0; i < njobs && ring; i++)
+        if (!ring_job(lut_from_handle(jobs[i].lut), jobs[i].radius, jobs[i].mode, cfg, halo, &dj[i])) {
+            set_error("job " + std::to_string(i) + ": template does not hold the unrolled kernel's taps");
+            return kInvalidData;
+        }
     for (int i = 0; i < njobs; i++) max_lut_rows = std::max(max_lut_rows, dj[i].lut_rows);
     if (lds_bytes(cfg, halo, max_lut_rows) > max_lds_bytes()) {
         set_error("tile config does not fit the weight tables in LDS");
