@@ -149,7 +149,8 @@ int64_t bf_batch_pixels(bf_batch batch);
 int bf_batch_config(bf_batch batch);
 /* 1 when every job uses the canonical GAUSS-factory template at a radius
  * with an unrolled batch kernel (1 to 16) and the batch runs those
- * kernels (tile configs 0 and 1), 0 when it runs the tap-list kernel,
+ * kernels (tile configs 0 and 1; not on config 1 where REF jobs of r = 16
+ * are more than a third of the work), 0 when it runs the tap-list kernel,
  * < 0 on error.  Same output bits either way. */
 int bf_batch_unrolled(bf_batch batch);
 

@@ -775,6 +775,7 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
     std::vector<int64_t> cost(njobs);
     int max_rows = 0, max_lut_rows = 0;
     int64_t pixels = 0;
+    double work = 0.0, work_ref16 = 0.0;      // pixel-taps, of all jobs and of REF r = 16
     for (int i = 0; i < njobs; i++) {
         int64_t px = 0;
         if (!jobs[i].lut) {
@@ -794,13 +795,23 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
         max_rows = std::max(max_rows, dj[i].nrows);
         cost[i] = (int64_t)dj[i].ntaps_padded;
         pixels += px;
+        work += (double)px * cost[i];
+        if (jobs[i].mode == BF_MODE_REF && jobs[i].radius == 16) work_ref16 += (double)px * cost[i];
     }
+    // REF r = 16 on 64 x 32 tiles: the unrolled kernel's table leaves one
+    // eight-wave workgroup a CU, and the tap list, whose table is 1 KB there, is
+    // faster (4096 x 2048, us: 1,104 against 1,336), while every other radius
+    // and mode gains from the unrolled kernels (3 to 22%): the tap list where
+    // these jobs are more than a third of the work.
+    const bool canonical = all_canonical(jobs, njobs);
+    auto unrolled = [&](int c) {
+        return canonical && ring_batch_supported(c, halo) && !(c == 1 && 3.0 * work_ref16 > work);
+    };
     // The unrolled kernels take what fits in LDS of a table beside any of their
     // tiles, and costs of the canonical template were measured with its table
     // as it runs beside a tile; only otherwise a configuration has to be found
     // beside which the tables fit.
-    const bool canonical = all_canonical(jobs, njobs);
-    if (config < 0 && !(canonical && (tuned || ring_batch_supported(cfg, halo)))) {
+    if (config < 0 && !unrolled(cfg) && !(canonical && tuned)) {
         const int c = fit_config(cfg, rmax, max_rows);
         if (c != cfg) {   // re-plan the jobs with the configuration that fits
             cfg = c;
@@ -813,7 +824,7 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
     }
     // All on the canonical template, on tiles with unrolled kernels: those, with
     // their per-q tables.
-    const bool ring = canonical && ring_batch_supported(cfg, halo);
+    const bool ring = unrolled(cfg);
     for (int i = 0; i < njobs && ring; i++)
         if (!ring_job(lut_from_handle(jobs[i].lut), jobs[i].radius, jobs[i].mode, cfg, halo, &dj[i])) {
             set_error("job " + std::to_string(i) + ": template does not hold the unrolled kernel's taps");

@@ -65,11 +65,22 @@ def test_r16_takes_the_measured_configuration(device, tuned, mode, config):
     tuned.install(16, mode, cost)
     b = _Batch([(16, mode)])
     assert b.batch.config == config
-    assert b.batch.unrolled == (config in (0, 1))
+    assert b.batch.unrolled == (config == 0 or (config == 1 and mode == STD))
     b.check()
 
 
 def test_custom_template_keeps_a_configuration_its_table_fits(device, tuned):
     b = _Batch([(16, STD)], custom=True)
     assert not b.batch.unrolled and b.batch.config == 2
+    b.check()
+
+
+@pytest.mark.parametrize("pairs,unrolled", [([(16, REF)], False), ([(16, STD)], True), ([(15, REF)], True),
+                                            ([(16, REF), (16, STD)], False),
+                                            ([(16, REF), (15, REF), (16, STD)], False),
+                                            ([(16, REF), (15, REF), (16, STD), (14, STD)], True)])
+def test_ref_r16_on_64x32_tiles(device, pairs, unrolled):
+    # the tap list where REF r = 16 is more than a third of the pixel-taps
+    b = _Batch(pairs, config=1)
+    assert b.batch.unrolled == unrolled
     b.check()
