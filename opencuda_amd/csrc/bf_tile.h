@@ -297,12 +297,14 @@ constexpr int ring_fused_rows()
 //   STD r = 13, 15: 447, 579 at 20; 444, 581 at 40; 447, 592 at 48;
 //   STD r = 18: 838 at 36, 841 at 30, 868 at 28, 855 at 52.
 // The batch kernel holds both modes and keeps to windows whose registers
-// leave two workgroups a CU (BATCH).
+// leave two workgroups a CU (BATCH), six waves a SIMD to r = 8: STD r = 5, 7
+// on 64 x 32 tiles of 4096 x 2048: 161.0, 269.2 at 24 taps, 158.7, 267.2 at 28,
+// 156.5, 265.9 at 32 (r = 6 and 4 then slower), 161.0, 285.9 at 36.
 template <int MODE, int HALO, bool BATCH>
 constexpr int ring_group()
 {
     if (MODE == kModeRef) return 4;
-    if (BATCH) return HALO <= 12 ? 24 : 40;
+    if (BATCH) return HALO <= 8 ? 28 : (HALO <= 12 ? 24 : 40);
     return HALO <= 4 ? 28 : (HALO <= 12 ? 60 : (HALO <= 16 ? 20 : 36));
 }
 
