@@ -157,24 +157,31 @@ int bf_batch_unrolled(bf_batch batch);
 /* Autotuner (no reference counterpart).  bf_tune_radius times every tile
  * configuration (tile shape and columns per lane, bf_tune_describe) for
  * (radius, mode) on the current device -- a synthetic width x height image,
- * sigma_space = radius/1.5, sigma_range = 30, run as a one-job batch with
- * that configuration (so the unrolled kernels are timed where a batch would
- * use them), `reps` timed launches after one warm-up -- and installs the
- * fastest in a process-wide table.  bf_exact (where it runs the tap-list kernel) and
- * bf_batch_create (config < 0) use that
- * table: a single image takes the tuned configuration of its radius; a
- * batch whose radii are all tuned takes the configuration with the least
- * estimated total time (sum over jobs of pixels x measured cost).
- *   best_config: receives the winner; ms_per_mpix (bf_tune_count() floats,
- *   may be NULL): measured cost of each configuration, < 0 if it could not
- *   run.  Synchronous. */
+ * sigma_space = radius/1.5, sigma_range = 30, run as a one-job batch on the
+ * canonical template, as the same on the tap-list kernel and as
+ * bf_exact_config, in turns, the best of `reps` launches each -- and installs
+ * the costs in a process-wide table.  bf_exact, where it runs the tap-list
+ * kernel, takes the configuration with the least cost there (the built-in
+ * default within 3% of it; a smaller tile where the image fills too few of the
+ * device's CUs); bf_batch_create (config < 0), when all its radii are tuned,
+ * the one with the least estimated total time (sum over jobs of pixels x the
+ * cost of a batch on the kernel it would run; the default within 2% of it).
+ *   best_config: receives the best for a batch on the canonical template;
+ *   ms_per_mpix (bf_tune_count() floats, may be NULL): its measured cost with
+ *   each configuration, < 0 if it could not run.  Synchronous. */
 int bf_tune_radius(int32_t radius, int32_t mode, int32_t width, int32_t height,
                    int32_t reps, int32_t *best_config, float *ms_per_mpix);
 /* Install / read a table entry (e.g. from a saved tuning run):
  * ms_per_mpix as above.  bf_tune_get returns the tuned configuration, or
- * -1 if (radius, mode) has not been tuned. */
+ * -1 if (radius, mode) has not been tuned.  bf_tune_set takes the costs for
+ * all launches; bf_tune_set_taps then gives the tap-list kernel its own, for one
+ * image and for a batch (an error where the entry has not been set), and
+ * bf_tune_get_taps reads them (either may be NULL) and returns the best for one
+ * image. */
 int bf_tune_set(int32_t radius, int32_t mode, const float *ms_per_mpix);
 int bf_tune_get(int32_t radius, int32_t mode, float *ms_per_mpix);
+int bf_tune_set_taps(int32_t radius, int32_t mode, const float *single, const float *batch);
+int bf_tune_get_taps(int32_t radius, int32_t mode, float *single, float *batch);
 /* Forget every tuned entry (back to the built-in defaults). */
 int bf_tune_reset(void);
 

@@ -86,6 +86,8 @@ def lib() -> ctypes.CDLL:
         "bf_tune_radius": ([I32, I32, I32, I32, I32, P, P], ctypes.c_int),
         "bf_tune_set": ([I32, I32, P], ctypes.c_int),
         "bf_tune_get": ([I32, I32, P], ctypes.c_int),
+        "bf_tune_set_taps": ([I32, I32, P, P], ctypes.c_int),
+        "bf_tune_get_taps": ([I32, I32, P, P], ctypes.c_int),
         "bf_tune_reset": ([], ctypes.c_int),
         "bf_batch_create": ([P, I32, I32, ctypes.POINTER(P)], ctypes.c_int),
         "bf_batch_destroy": ([P], ctypes.c_int),

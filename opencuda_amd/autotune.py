@@ -2,11 +2,15 @@
 columns per lane (bf_tune_radius, bf_tune_describe).
 
 For each (radius, mode) the library times every tile configuration on the
-device and keeps the fastest in a process-wide table that bf_exact and
-bf_batch_create consult (a batch picks the configuration with the least
-estimated total time over its jobs).  Tables can be saved to JSON and
-installed again in a later process (bf_tune_set).  `tune_batch` times a
-given batch itself with every configuration.
+device, for a batch on the canonical template (the unrolled kernels where it
+runs those), for one on the tap-list kernel and for one image there, and keeps
+the costs in a process-wide table.  bf_batch_create
+picks the configuration with the least estimated total time over its jobs, and
+bf_exact the best of the tap-list kernel where it runs that (other templates
+than the canonical one; its unrolled kernels have tiles of their own rule).
+Tables can be saved to JSON and installed again in a later process
+(bf_tune_set, bf_tune_set_taps).  `tune_batch` times a given batch itself with
+every configuration.
 
     python -m opencuda_amd.autotune --out opencuda_amd/data/tune_gfx950.json
 """
@@ -43,17 +47,34 @@ def tune(radius: int, mode: int, width: int = 4096, height: int = 2048, reps: in
     return best.value, [float(c) for c in cost]
 
 
-def install(radius: int, mode: int, ms_per_mpix) -> None:
+def install(radius: int, mode: int, ms_per_mpix, taps=None, batch_taps=None) -> None:
+    """Costs of the configurations for a batch on the canonical template; taps,
+    batch_taps: of the tap-list kernel for one image and for a batch (default:
+    the same)."""
     from . import _check
     c = np.ascontiguousarray(ms_per_mpix, np.float32)
     assert c.size == _nconf()
     _check(_lib().bf_tune_set(int(radius), int(mode), c.ctypes.data), "bf_tune_set")
+    if taps is not None or batch_taps is not None:
+        t = np.ascontiguousarray(ms_per_mpix if taps is None else taps, np.float32)
+        b = np.ascontiguousarray(ms_per_mpix if batch_taps is None else batch_taps, np.float32)
+        assert t.size == b.size == _nconf()
+        _check(_lib().bf_tune_set_taps(int(radius), int(mode), t.ctypes.data, b.ctypes.data),
+               "bf_tune_set_taps")
 
 
 def get(radius: int, mode: int):
     cost = np.zeros(_nconf(), np.float32)
     best = int(_lib().bf_tune_get(int(radius), int(mode), cost.ctypes.data))
     return (best, [float(c) for c in cost]) if best >= 0 else (-1, None)
+
+
+def get_taps(radius: int, mode: int):
+    """(best configuration of one image, its costs, a batch's) on the tap-list
+    kernel."""
+    one, many = np.zeros(_nconf(), np.float32), np.zeros(_nconf(), np.float32)
+    best = int(_lib().bf_tune_get_taps(int(radius), int(mode), one.ctypes.data, many.ctypes.data))
+    return (best, [float(c) for c in one], [float(c) for c in many]) if best >= 0 else (-1, None, None)
 
 
 def reset() -> None:
@@ -94,7 +115,9 @@ def tune_all(radii=(3, 5, 7, 9, 15), modes=(0, 1), width=4096, height=2048, reps
     for mode in modes:
         for r in radii:
             best, cost = tune(r, mode, width, height, reps)
-            table[f"{mode}:{r}"] = {"best": best, "ms_per_mpix": cost}
+            _, taps, batch_taps = get_taps(r, mode)
+            table[f"{mode}:{r}"] = {"best": best, "ms_per_mpix": cost, "taps_ms_per_mpix": taps,
+                                    "batch_taps_ms_per_mpix": batch_taps}
             if log:
                 log(f"mode {mode} r {r}: best config {best}, ms/Mpix {[round(c, 4) for c in cost]}")
     return table
@@ -118,7 +141,8 @@ def load(path: str = DEFAULT_TABLE) -> int:
     n = 0
     for key, ent in doc["entries"].items():
         mode, r = (int(v) for v in key.split(":"))
-        install(r, mode, ent["ms_per_mpix"])
+        install(r, mode, ent["ms_per_mpix"], ent.get("taps_ms_per_mpix"),
+                ent.get("batch_taps_ms_per_mpix"))
         n += 1
     return n
 

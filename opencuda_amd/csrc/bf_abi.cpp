@@ -85,11 +85,16 @@ struct LutFull : Lut {
 Lut *lut_from_handle(bf_lut h) { return reinterpret_cast<Lut *>(h); }
 
 // Autotuner results: measured ms per Mpix of each tile configuration for
-// (mode, radius); an entry is "tuned" when at least one cost is >= 0.
+// (mode, radius), of a batch on the canonical template (cost: the unrolled
+// kernels where they apply), of a tap-list launch of one image (taps) and of a
+// tap-list batch (batch_taps); an entry is "tuned" when at least one cost is
+// >= 0.
 struct TuneTable {
     std::mutex mu;
     bool have[2][BF_MAX_RADIUS + 1] = {};
     float cost[2][BF_MAX_RADIUS + 1][16] = {};
+    float taps[2][BF_MAX_RADIUS + 1][16] = {};
+    float batch_taps[2][BF_MAX_RADIUS + 1][16] = {};
 };
 
 static TuneTable &tune_table()
@@ -98,17 +103,20 @@ static TuneTable &tune_table()
     return *t;
 }
 
-// Tuned configuration for (radius, mode), or -1.
-static int tuned_config(int radius, int mode)
+// Tuned configuration for (radius, mode), of one image on the tap-list kernel or
+// of a batch on the canonical template, or -1; copies the costs where `costs`
+// is set.
+static int tuned_config(int radius, int mode, bool taps, float *costs = nullptr)
 {
     if (radius < 1 || radius > BF_MAX_RADIUS || (mode != 0 && mode != 1)) return -1;
     TuneTable &t = tune_table();
     std::lock_guard<std::mutex> lock(t.mu);
     if (!t.have[mode][radius]) return -1;
+    const float *k = taps ? t.taps[mode][radius] : t.cost[mode][radius];
     int best = -1;
     for (int c = 0; c < tile_config_count(); c++)
-        if (t.cost[mode][radius][c] >= 0 && (best < 0 || t.cost[mode][radius][c] < t.cost[mode][radius][best]))
-            best = c;
+        if (k[c] >= 0 && (best < 0 || k[c] < k[best])) best = c;
+    if (best >= 0 && costs) std::copy(k, k + tile_config_count(), costs);
     return best;
 }
 
@@ -252,6 +260,10 @@ bool views_overlap(const bf_image_view *a, const bf_image_view *b)
 }  // namespace bfimpl
 
 using namespace bfimpl;
+
+namespace {
+int create_batch(const bf_job *jobs, int njobs, int config, bool tap_list, bf_batch *out);
+}
 
 extern "C" {
 
@@ -482,9 +494,38 @@ static ExactPlan plan_exact(const Lut *L, int radius, int mode, int W, int H)
         if (config >= 0) return { config, true };
     }
     const int rows = fused_rows(L, radius, mode);
-    const int tuned = tuned_config(radius, mode);
-    const int want = tuned >= 0 ? tuned : (radius >= 17 ? 3 : default_config(radius, mode));
-    return { rows < 0 ? default_config(1, mode) : fit_config(want, radius, rows), false };
+    // The table's costs are those of a large image; a small one takes as long as
+    // its fullest CU.  Where a configuration's cost times the pixels of the tiles
+    // there is a tenth below that of the one with the least cost, it is taken
+    // (STD r = 6, us, 1021 x 767: 64 x 16 tiles 30, 128 x 16 34; at less than a
+    // tenth the estimate errs: REF r = 8, 0.97, 53 against 45).
+    // The built-in default stands where it is within 3% of the least cost: the
+    // order of such configurations changes with the image.
+    float cost[16];
+    const int normal = radius >= 17 ? 3 : default_config(radius, mode);
+    int tuned = tuned_config(radius, mode, true, cost), dev = 0, cus = 0;
+    if (tuned >= 0 && cost[normal] >= 0 && 0.97f * cost[normal] <= cost[tuned]) tuned = normal;
+    if (tuned >= 0 && hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0) {
+        auto estimate = [&](int c) {
+            const TileConfig &tc = tile_config(c);
+            const int th = 4 * tc.tgy;
+            const int64_t tiles = (int64_t)((W + tc.tw - 1) / tc.tw) * ((H + th - 1) / th);
+            return (double)cost[c] * tc.tw * th * (double)((tiles + cus - 1) / cus);
+        };
+        double least = 0.9 * estimate(tuned);
+        for (int c = 0; c < tile_config_count(); c++)
+            if (cost[c] >= 0 && estimate(c) < least) {
+                least = estimate(c);
+                tuned = c;
+            }
+    }
+    const int want = tuned >= 0 ? tuned : normal;
+    if (rows < 0) return { default_config(1, mode), false };
+    // a tuned cost was measured with a table of the canonical template's rows,
+    // in LDS as a whole or not: fewer run there no slower
+    const bool as_measured = tuned >= 0 && rows <= ring_rows(radius, mode);
+    return { as_measured ? want : fit_config(want, radius, rows), false };
 }
 
 int bf_exact(const bf_image_view *in, const bf_image_view *out, bf_lut lut, int32_t radius,
@@ -536,6 +577,9 @@ int bf_exact_plan(bf_lut lut, int32_t radius, int32_t mode, int32_t width, int32
     return plan.config;
 }
 
+// Turns of every configuration before the timed ones: some 20 launches.
+constexpr int kTuneWarmups = 2;
+
 int bf_tune_radius(int32_t radius, int32_t mode, int32_t width, int32_t height, int32_t reps,
                    int32_t *best_config, float *ms_per_mpix)
 {
@@ -557,7 +601,7 @@ int bf_tune_radius(int32_t radius, int32_t mode, int32_t width, int32_t height, 
     if (rc) return rc;
     unsigned char *din = nullptr, *dout = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    std::vector<float> cost(nc, -1.0f);
+    std::vector<float> cost(nc), taps(nc), batch_taps(nc);
     hipError_t e = hipMalloc(&din, host.size());
     if (e == hipSuccess) e = hipMalloc(&dout, host.size());
     if (e == hipSuccess) e = hipMemcpy(din, host.data(), host.size(), hipMemcpyHostToDevice);
@@ -565,29 +609,50 @@ int bf_tune_radius(int32_t radius, int32_t mode, int32_t width, int32_t height, 
     if (e == hipSuccess) e = hipEventCreate(&e1);
     if (e != hipSuccess) rc = hip_fail(e, "bf_tune_radius");
     bf_image_view vin{ din, width, height, width }, vout{ dout, width, height, width };
-    // Each configuration is timed as a one-job batch: the launch a batch
-    // with that configuration makes (the unrolled kernels where they apply,
-    // configurations 0 and 1 to r = 16; the tap-list kernel
-    // otherwise), which is what the table's costs steer.
+    // Each configuration is timed as a one-job batch, the launch a batch with
+    // that configuration makes, as the same on the tap-list kernel (where that
+    // is another) and as bf_exact's tap-list launch.  They take turns, a launch each, and keep their best: the clock still rises during
+    // the first launches (timed one after another from a cold start, the first
+    // two configurations came out 15% slower than they are).
     const bf_job job{ vin, vout, lut, radius, mode };
+    std::vector<bf_batch> batches(nc, nullptr), tap_batches(nc, nullptr);
     for (int c = 0; c < nc && rc == kOk; c++) {
-        bf_batch b = nullptr;
-        if (bf_batch_create(&job, 1, c, &b) != kOk) continue;
-        int r2 = bf_batch_run(b, nullptr);
-        if (r2 == kOk) {
-            hipEventRecord(e0, nullptr);
-            for (int k = 0; k < reps && r2 == kOk; k++) r2 = bf_batch_run(b, nullptr);
-            hipEventRecord(e1, nullptr);
-        }
+        if (create_batch(&job, 1, c, false, &batches[c]) != kOk) batches[c] = nullptr;
+        if (batches[c] && bf_batch_unrolled(batches[c]) == 1 &&
+            create_batch(&job, 1, c, true, &tap_batches[c]) != kOk)
+            tap_batches[c] = nullptr;
+    }
+    auto time_launch = [&](auto launch, float *best) {
+        hipEventRecord(e0, nullptr);
+        const int r2 = launch();
+        hipEventRecord(e1, nullptr);
         if (hipEventSynchronize(e1) != hipSuccess) {
-            bf_batch_destroy(b);
             rc = kHipError;
-            break;
+            return;
         }
-        bf_batch_destroy(b);
         float ms = 0.0f;
         hipEventElapsedTime(&ms, e0, e1);
-        if (r2 == kOk) cost[c] = ms / reps / ((float)width * height / 1e6f);
+        ms /= (float)width * height / 1e6f;
+        if (r2 == kOk && (*best < 0 || ms < *best)) *best = ms;
+    };
+    for (int k = -kTuneWarmups; k < reps && rc == kOk; k++) {
+        if (k == 0) {
+            std::fill(cost.begin(), cost.end(), -1.0f);
+            std::fill(taps.begin(), taps.end(), -1.0f);
+            std::fill(batch_taps.begin(), batch_taps.end(), -1.0f);
+        }
+        for (int c = 0; c < nc && rc == kOk; c++) {
+            if (batches[c]) time_launch([&] { return bf_batch_run(batches[c], nullptr); }, &cost[c]);
+            if (tap_batches[c] && rc == kOk)
+                time_launch([&] { return bf_batch_run(tap_batches[c], nullptr); }, &batch_taps[c]);
+            if (rc == kOk)
+                time_launch([&] { return bf_exact_config(&vin, &vout, lut, radius, mode, c, nullptr); }, &taps[c]);
+        }
+    }
+    for (int c = 0; c < nc; c++) {
+        if (!tap_batches[c] && !(batches[c] && bf_batch_unrolled(batches[c]) == 1)) batch_taps[c] = cost[c];
+        if (batches[c]) bf_batch_destroy(batches[c]);
+        if (tap_batches[c]) bf_batch_destroy(tap_batches[c]);
     }
     if (e0) hipEventDestroy(e0);
     if (e1) hipEventDestroy(e1);
@@ -596,8 +661,9 @@ int bf_tune_radius(int32_t radius, int32_t mode, int32_t width, int32_t height, 
     bf_lut_destroy(lut);
     if (rc) return rc;
     int rc2 = bf_tune_set(radius, mode, cost.data());
+    if (rc2 == kOk) rc2 = bf_tune_set_taps(radius, mode, taps.data(), batch_taps.data());
     if (rc2) return rc2;
-    if (best_config) *best_config = tuned_config(radius, mode);
+    if (best_config) *best_config = tuned_config(radius, mode, false);
     if (ms_per_mpix) std::copy(cost.begin(), cost.end(), ms_per_mpix);
     return kOk;
 }
@@ -610,21 +676,42 @@ int bf_tune_set(int32_t radius, int32_t mode, const float *ms_per_mpix)
     std::lock_guard<std::mutex> lock(t.mu);
     bool any = false;
     for (int c = 0; c < tile_config_count(); c++) {
-        t.cost[mode][radius][c] = ms_per_mpix[c];
+        t.cost[mode][radius][c] = t.taps[mode][radius][c] = t.batch_taps[mode][radius][c] = ms_per_mpix[c];
         any = any || ms_per_mpix[c] >= 0;
     }
     t.have[mode][radius] = any;
     return kOk;
 }
 
+int bf_tune_set_taps(int32_t radius, int32_t mode, const float *single, const float *batch)
+{
+    if (!single || !batch) return kNullPointer;
+    if (radius < 1 || radius > BF_MAX_RADIUS || (mode != 0 && mode != 1)) return kInvalidData;
+    TuneTable &t = tune_table();
+    std::lock_guard<std::mutex> lock(t.mu);
+    if (!t.have[mode][radius]) {
+        set_error("no tuned entry for this radius and mode");
+        return kInvalidData;
+    }
+    std::copy(single, single + tile_config_count(), t.taps[mode][radius]);
+    std::copy(batch, batch + tile_config_count(), t.batch_taps[mode][radius]);
+    return kOk;
+}
+
 int bf_tune_get(int32_t radius, int32_t mode, float *ms_per_mpix)
 {
     if (radius < 1 || radius > BF_MAX_RADIUS || (mode != 0 && mode != 1)) return kInvalidData;
-    const int best = tuned_config(radius, mode);
-    if (best >= 0 && ms_per_mpix) {
+    return tuned_config(radius, mode, false, ms_per_mpix);
+}
+
+int bf_tune_get_taps(int32_t radius, int32_t mode, float *single, float *batch)
+{
+    if (radius < 1 || radius > BF_MAX_RADIUS || (mode != 0 && mode != 1)) return kInvalidData;
+    const int best = tuned_config(radius, mode, true, single);
+    if (best >= 0 && batch) {
         TuneTable &t = tune_table();
         std::lock_guard<std::mutex> lock(t.mu);
-        for (int c = 0; c < tile_config_count(); c++) ms_per_mpix[c] = t.cost[mode][radius][c];
+        std::copy(t.batch_taps[mode][radius], t.batch_taps[mode][radius] + tile_config_count(), batch);
     }
     return best;
 }
@@ -703,8 +790,10 @@ struct Batch {
 
 }  // namespace bfimpl
 
+namespace {
+
 // Every job on the canonical template and within its taps.
-static bool all_canonical(const bf_job *jobs, int njobs)
+bool all_canonical(const bf_job *jobs, int njobs)
 {
     for (int i = 0; i < njobs; i++) {
         const Lut *L = lut_from_handle(jobs[i].lut);
@@ -715,9 +804,8 @@ static bool all_canonical(const bf_job *jobs, int njobs)
     return true;
 }
 
-extern "C" {
-
-int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch *out)
+// bf_batch_create, or the same with the tap-list kernel whatever the template.
+int create_batch(const bf_job *jobs, int njobs, int config, bool tap_list, bf_batch *out)
 {
     if (!jobs || !out) {
         set_error("null argument");
@@ -734,10 +822,30 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
         return kInvalidData;
     }
     const int halo = halo_class(rmax);
+    // Pixel-taps, of all jobs and of REF r = 16.  REF r = 16 on 64 x 32 tiles: the
+    // unrolled kernel's table leaves one eight-wave workgroup a CU, and the tap
+    // list, whose table is 1 KB there, is faster (4096 x 2048, us: 1,104 against
+    // 1,336), while every other radius and mode gains from the unrolled kernels
+    // (3 to 22%): the tap list where these jobs are more than a third of the work.
+    double work = 0.0, work_ref16 = 0.0;
+    for (int i = 0; i < njobs; i++) {
+        const double side = 2.0 * jobs[i].radius + 1.0;
+        const double w = (double)std::min(jobs[i].in.width, jobs[i].out.width) *
+                         std::min(jobs[i].in.height, jobs[i].out.height) * side * side;
+        work += w;
+        if (jobs[i].mode == BF_MODE_REF && jobs[i].radius == 16) work_ref16 += w;
+    }
+    const bool canonical = !tap_list && all_canonical(jobs, njobs);
+    auto unrolled = [&](int c) {
+        return canonical && ring_batch_supported(c, halo) && !(c == 1 && 3.0 * work_ref16 > work);
+    };
     // Validate and size every job with a provisional config: the one with
     // the least estimated time when every (radius, mode) is tuned, else the
-    // built-in default for the largest radius.
-    int cfg = config >= 0 ? config : default_config(rmax, jobs[0].mode);
+    // built-in default for the largest radius, which also stands within 2% of
+    // the least (costs are of one radius with its own halo: STD r = 15 and 7,
+    // estimates 0.987 for 64 x 32 against 64 x 64 tiles, 1,532 against 1,456 us).
+    const int normal = default_config(rmax, jobs[0].mode);
+    int cfg = config >= 0 ? config : normal;
     bool tuned = false;
     if (config < 0) {
         TuneTable &t = tune_table();
@@ -748,12 +856,13 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
             all = r >= 1 && r <= BF_MAX_RADIUS && (m == 0 || m == 1) && t.have[m][r];
         }
         if (all) {
-            double best = -1.0;
+            double best = -1.0, at_default = -1.0;
             for (int c = 0; c < tile_config_count(); c++) {
                 double est = 0.0;
                 bool ok = true;
                 for (int i = 0; i < njobs && ok; i++) {
-                    const float k = t.cost[jobs[i].mode][jobs[i].radius][c];
+                    const int r = jobs[i].radius, m = jobs[i].mode;
+                    const float k = unrolled(c) ? t.cost[m][r][c] : t.batch_taps[m][r][c];
                     if (k < 0) ok = false;
                     const double px = (double)std::min(jobs[i].in.width, jobs[i].out.width) *
                                       std::min(jobs[i].in.height, jobs[i].out.height);
@@ -764,7 +873,9 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
                     cfg = c;
                     tuned = true;
                 }
+                if (ok && c == normal) at_default = est;
             }
+            if (at_default >= 0 && 0.98 * at_default <= best) cfg = normal;
         }
     }
     if (cfg >= tile_config_count()) {
@@ -774,8 +885,8 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
     std::vector<DevJob> dj(njobs);
     std::vector<int64_t> cost(njobs);
     int max_rows = 0, max_lut_rows = 0;
+    bool as_measured = tuned;
     int64_t pixels = 0;
-    double work = 0.0, work_ref16 = 0.0;      // pixel-taps, of all jobs and of REF r = 16
     for (int i = 0; i < njobs; i++) {
         int64_t px = 0;
         if (!jobs[i].lut) {
@@ -793,25 +904,15 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
             return rc;
         }
         max_rows = std::max(max_rows, dj[i].nrows);
+        as_measured = as_measured && dj[i].nrows <= ring_rows(jobs[i].radius, jobs[i].mode);
         cost[i] = (int64_t)dj[i].ntaps_padded;
         pixels += px;
-        work += (double)px * cost[i];
-        if (jobs[i].mode == BF_MODE_REF && jobs[i].radius == 16) work_ref16 += (double)px * cost[i];
     }
-    // REF r = 16 on 64 x 32 tiles: the unrolled kernel's table leaves one
-    // eight-wave workgroup a CU, and the tap list, whose table is 1 KB there, is
-    // faster (4096 x 2048, us: 1,104 against 1,336), while every other radius
-    // and mode gains from the unrolled kernels (3 to 22%): the tap list where
-    // these jobs are more than a third of the work.
-    const bool canonical = all_canonical(jobs, njobs);
-    auto unrolled = [&](int c) {
-        return canonical && ring_batch_supported(c, halo) && !(c == 1 && 3.0 * work_ref16 > work);
-    };
     // The unrolled kernels take what fits in LDS of a table beside any of their
-    // tiles, and costs of the canonical template were measured with its table
-    // as it runs beside a tile; only otherwise a configuration has to be found
-    // beside which the tables fit.
-    if (config < 0 && !unrolled(cfg) && !(canonical && tuned)) {
+    // tiles, and tuned costs were measured with the canonical table as it runs
+    // beside a tile; only otherwise a configuration has to be found beside which
+    // the tables fit.
+    if (config < 0 && !unrolled(cfg) && !as_measured) {
         const int c = fit_config(cfg, rmax, max_rows);
         if (c != cfg) {   // re-plan the jobs with the configuration that fits
             cfg = c;
@@ -874,6 +975,15 @@ int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch 
     }
     *out = reinterpret_cast<bf_batch>(B);
     return kOk;
+}
+
+}  // namespace
+
+extern "C" {
+
+int bf_batch_create(const bf_job *jobs, int32_t njobs, int32_t config, bf_batch *out)
+{
+    return create_batch(jobs, njobs, config, false, out);
 }
 
 int bf_batch_config(bf_batch h)
