@@ -277,8 +277,9 @@ constexpr int ring_min_offset()
 }
 
 // Rows of the fused table a workgroup's LDS holds beside its tile and one
-// more row.  Radii with more rows (17 and up, and 16 on 64 x 64 tiles) keep
-// the first ones fused; a tap of any other row reads E[d] from that last row
+// more row.  Radii with more rows (16 and up: 135 or 136 rows at r = 16 against
+// 122 beside 64 x 64 tiles and 134 beside 64 x 32 ones) keep the first ones
+// fused; a tap of any other row reads E[d] from that last row
 // and forms the factor g * E[d] itself, the product the fused rows hold,
 // with the same single rounding.
 template <int TW, int TGY, int HALO>

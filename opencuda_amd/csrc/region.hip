@@ -2,25 +2,31 @@
 // okano_3_0/SimpleRegionDetect.cu:287-312: LocalCluster before it and
 // ConnectRegion after it, for gfx950.
 //
-// LocalCluster (okano_3_0/LocalCluster.cu:45-153): one lane per pixel runs
-// the eight directional walks the reference spreads over eight threads and
-// a shared array, with the same FP32 operations in the same order
-// (-ffp-contract=off, IEEE division), so the u8 result is the reference's.
+// LocalCluster (okano_3_0/LocalCluster.cu:45-153): the reference spreads a
+// pixel's eight directional walks over eight threads and a shared array.  Here
+// one lane per pixel makes the walks' first step, which settles most pixels,
+// and eight lanes run the walks of each other one; the averages are formed and
+// summed with the same FP32 operations in the same order (-ffp-contract=off,
+// IEEE division), so the u8 result is the reference's.
 // The reference addresses every read as data + y * pitch + x from the ROI
 // origin and its walks reach 2 (pntRange - 1) pixels from the centre while
 // the guard band is pntRange + 2 wide; reads here use the same linear
 // address, clamped into the allocation the caller declares.  A workgroup
-// stages its 64 x 16 tile plus the walks' reach in LDS by that rule.
+// stages its tile of 64 columns and 16, 32 or 64 rows plus the walks' reach in
+// LDS by that rule; for reaches too large for LDS one lane walks all eight
+// directions of a pixel in global memory.
 //
 // ConnectRegion (okano_3_0/ConnectRegion.cu:789-1043): 8-connected
 // components of pixels whose gray values lie in [minGray, maxGray], each
 // labelled by its minimum raster index.  The reference gets there with
-// shared-memory labelling per block and rounds of border merging; here each
-// 64 x 64 tile is labelled in LDS, then the runs that touch across tile
-// edges are joined by a lock-free union-find pass in global memory
-// (atomicMin on roots, parents always smaller than children, so every loop
-// ends), then path compression -- the result does not depend on the order
-// the unions run in.  Areas, the area filter, the raster-order
+// shared-memory labelling per block and rounds of border merging; here the
+// runs of each 64 x 64 tile are labelled in LDS, which leaves a handful of
+// tile-local roots, then the runs that touch across tile edges join those by a
+// lock-free union-find pass in global memory (atomicMin on roots, parents
+// always smaller than children, so every loop ends), then each tile-local root
+// is pointed at its global root and its area added there -- the result does
+// not depend on the order the unions run in.  No pass keeps a label per pixel.
+// The area filter, the raster-order
 // renumbering and the u8 output follow the reference, including its area
 // launch covering only rows below 256 * ceil(floor((H + 4) / 32) / 8)
 // (ConnectRegion.cu:45, :957-967) and never dropping a root whose counted

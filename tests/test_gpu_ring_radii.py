@@ -86,8 +86,9 @@ def test_surrogate_check_and_fallback(device, r, mode):
                                    (17, 1100, 1000), (18, 1100, 1000),
                                    (3, 1021, 767), (4, 1100, 1000), (7, 1021, 767), (8, 1700, 1300)])
 def test_images_past_the_small_tiles(device, r, w, h, mode):
-    # r > 9: the 64 x 64 kernels (203 x 139 above: 64 x 32); r <= 8: several
-    # rounds of 64 x 16 tiles, and 64 x 32 tiles at 1700 x 1300 (203 x 139: one)
+    # Images of several rounds of tiles.  Which kernel an image takes, and every
+    # kernel at sizes that take it: test_gpu_exact_plan.py.  (REF r = 17 and 18
+    # take the tap list themselves here.)
     ring, taps = _luts(r / 1.5, 30.0)
     img = _img(w, h, r)
     got = run_exact(img, r, 0, 0, mode, lut=ring)
